@@ -112,6 +112,7 @@ int apply_shape( nufi_batch *b, const launch_shape &s )
         h.p.chunk = trace1d_chunk( q, b->variant, s, 65536, &pipe );
         h.p.pipe = pipe ? 1u : 0u;
         lds = std::max( lds, ( pipe ? 2 : 1 ) * size_t( h.p.chunk ) * b->sq[r] * elem );
+        (void)trace1d_xm_setup( h.p, s, false, 0 );
         h.wg_begin = uint32_t( wg_run.size() );
         h.n_wg = trace1d_grid( h.p, b->variant, s );
         wg_run.insert( wg_run.end(), h.n_wg, uint32_t( r ) );
@@ -243,7 +244,7 @@ int nufi_batch_create( const nufi_config *confs, uint64_t n_runs, int order, int
         p.Nx = uint32_t( c.Nx ); p.Nu = uint32_t( c.Nu ); p.stride_d = b->sd[r];
         p.ix_first = 0; p.ix_count = uint32_t( c.Nx );
         p.order = uint32_t( order ); p.mode = MODE_RHO;
-        trace1d_xm_setup( p );
+        p.ppx = xm_ppx( p.Nu );
         p.x_min = c.x_min; p.dx = c.dx; p.dx_inv = c.dx_inv; p.Lx = c.Lx; p.Lx_inv = c.Lx_inv; p.dt = c.dt;
         p.nx_min = c.x_min; p.ndx = c.dx; p.nu_min = c.u_min; p.ndu = c.du;
         fp32c_frame( double( c.Nx ), c.dt * c.dx_inv, c.u_min, double( c.Nu ), c.du, p.f32_p0, p.f32_w0 );

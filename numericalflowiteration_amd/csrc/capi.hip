@@ -319,7 +319,7 @@ int launch_trace( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_end, uin
         fp32c_frame( double( c->conf.Nx ), c->conf.dt * c->conf.dx_inv, c->conf.u_min, double( c->conf.Nu ),
                      c->conf.du, p.f32_p0, p.f32_w0 );
         p.f0 = c->conf.f0;
-        e = launch_trace1d( p, c->variant, c->shape, c->stream );
+        e = launch_trace1d( p, c->variant, c->shape, c->n_cu, c->stream );
     }
     else
     {
@@ -667,7 +667,7 @@ int nufi_compute_metrics( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_
             p.weight = m.du * m.dx;                                // cuda_kernel.cu:71
             p.f0 = g.f0;
             const int chunk = int( std::max<size_t>( 1, std::min<size_t>( 64, std::min<size_t>( c->lds_cap, 65536 ) / ( size_t( c->sd ) * 8 ) ) ) );
-            e = launch_trace1d( p, variant, launch_shape { 256, 1, chunk }, c->stream );
+            e = launch_trace1d( p, variant, launch_shape { 256, 1, chunk }, c->n_cu, c->stream );
         }
         else
         {

@@ -33,13 +33,13 @@ enum trace_variant : int
 // wave-tasks; task g covers ix = ix_first + g / wpx and iu = (g % wpx)*64 +
 // lane, and writes one partial sum of f to partials[(g % wpx)*Nx + ix].
 //
-// x-major (fast and FP32C rho kernels): the 64 lanes of a wave take xw
-// consecutive x nodes (xw = min(Nx, 64)) at vpw = 64/xw velocities; lanes at
+// x-major (fast and FP32C rho kernels): the threads of a workgroup take xw
+// consecutive x nodes (x fastest, xw <= 64) at `rows` velocities; threads at
 // one velocity and neighbouring x stay close along their characteristics, so
 // the table reads of a wave are near-contiguous in LDS.  Workgroup b covers
 // x-tile b % n_xt (x nodes ix_first + xw*(b % n_xt) + 0..xw-1) and velocity
-// block b / n_xt of vb = NPT*WPB*vpw velocities; thread (wave w, lane) takes
-// the velocity rows (r*WPB + w)*vpw + lane/xw, r < NPT.  The f values are
+// block b / n_xt of NPT*rows velocities; thread t takes the velocity rows
+// r*rows + t/xw, r < NPT.  The f values are
 // staged in LDS and summed over fixed groups of XM_GROUP consecutive
 // velocities (a sequential compensated sum in iu order) into
 // partials[(iu/XM_GROUP)*Nx + ix], ppx = ceil(Nu/XM_GROUP) groups: the
@@ -47,7 +47,6 @@ enum trace_variant : int
 // group-major (partials[j*n_space + i]), so both their writers and the
 // field kernel's fixed-order sum over j read and write coalesced.
 constexpr uint32_t XM_GROUP = 16;
-inline uint32_t xm_xw( uint32_t Nx ) { return Nx < 64 ? Nx : 64; }
 inline uint32_t xm_ppx( uint32_t Nu ) { return ( Nu + XM_GROUP - 1 ) / XM_GROUP; }
 
 // Trace kernel outputs.
@@ -72,7 +71,7 @@ struct trace1_params
     uint64_t q_begin, q_end;
     uint32_t Nx, Nu, stride_d, wpx;   // Nu / wpx: of the node grid
     uint32_t ix_first, n_tasks;
-    uint32_t ix_count, xw, vpw, n_xt, ppx;   // x-major: x range, tile shape, partials per x
+    uint32_t ix_count, xw, rows, n_xt, ppx;  // x-major: x range, tile shape, partials per x
     uint32_t chunk;          // slices per LDS chunk
     uint32_t order;
     int      mode;           // trace_mode
@@ -194,9 +193,8 @@ struct launch_shape
 };
 
 // Launchers (trace1d.hip / trace3d.hip).  Return hipSuccess or the error.
-hipError_t launch_trace1d( const trace1_params &p, int variant, const launch_shape &s, hipStream_t st );
+hipError_t launch_trace1d( const trace1_params &p, int variant, const launch_shape &s, int n_cu, hipStream_t st );
 hipError_t launch_trace3d( const trace3_params &p, int variant, const launch_shape &s, hipStream_t st );
-size_t trace1d_lds_bytes( const trace1_params &p, int variant, const launch_shape &s );
 size_t trace1d_slice_elems( const trace1_params &p, int variant );
 hipError_t launch_trace1d_batch( const batch_run *runs, const uint32_t *wg_run, uint32_t n_wg, uint64_t n,
                                  int variant, const launch_shape &s, size_t lds, hipStream_t st );
@@ -213,14 +211,15 @@ inline bool fast3_dma( uint32_t chunk, uint32_t st )
     return 2ull * ( uint64_t( chunk ) * st + 2 ) * sizeof(double) <= 160u * 1024u;
 }
 bool trace1d_shape_ok( int variant, int order, const launch_shape &s );
-// x-major fields (xw, vpw, n_xt, ppx) from Nx, Nu and ix_count, the grid of
-// a launch (x-major or wave-task decomposition, by variant and mode) and the
+// x-major fields (xw, rows, n_xt, ppx) and the threads of a workgroup from Nu,
+// ix_count and the shape; the grid of a launch (x-major or wave-task decomposition, by variant and mode) and the
 // slices per LDS chunk it uses (bounded by the step and, x-major, planned by
 // poly_chunk_plan within lds_max bytes, *pipe telling which loop it takes)
-void trace1d_xm_setup( trace1_params &p );
+uint32_t trace1d_xm_setup( trace1_params &p, const launch_shape &s, bool spread, int n_cu );
 uint32_t trace1d_grid( const trace1_params &p, int variant, const launch_shape &s );
 uint32_t trace1d_chunk( const trace1_params &p, int variant, const launch_shape &s, size_t lds_max = 160 * 1024,
                         bool *pipe = nullptr );
+size_t trace1d_lds_bytes( const trace1_params &p, int variant, const launch_shape &s );
 bool trace3d_shape_ok( int variant, int order, const launch_shape &s );
 
 // ---- adjoint (adjoint1d.hip) ---------------------------------------------------

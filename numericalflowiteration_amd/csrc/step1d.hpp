@@ -220,9 +220,9 @@ __device__ __forceinline__ void put_poly( T *pair, T *q2p, double D0, double D1,
 // copied into the other by direct global->LDS loads, which take no registers
 // and no VALU; each wave waits for its own copies and the workgroup barrier
 // publishes them at the chunk's end, when chunk k's buffer is also free again.
-template <int BLOCK, typename T, typename STEPS>
+template <typename T, typename STEPS>
 __device__ __forceinline__ void poly_ready_pipeline( T *lds, const T *qhist, uint32_t sq, uint64_t n, uint32_t C,
-                                                     STEPS steps )
+                                                     uint32_t waves, STEPS steps )
 {
     if ( n == 0 ) return;
     const int Ci = int( C ), top = int( n ) - 1;
@@ -231,13 +231,13 @@ __device__ __forceinline__ void poly_ready_pipeline( T *lds, const T *qhist, uin
     auto lo_of  = [&]( int k ) { const int h = top - k * Ci; return h - Ci + 1 > 0 ? h - Ci + 1 : 0; };
     auto cnt_of = [&]( int k ) { return top - k * Ci - lo_of( k ) + 1; };
     T *const buf0 = lds, *const buf1 = lds + size_t( C ) * sq;
-    dma_copy16<BLOCK>( buf0, qhist + size_t( lo_of( 0 ) ) * sq, uint32_t( cnt_of( 0 ) ) * w16 );
+    dma_copy16( buf0, qhist + size_t( lo_of( 0 ) ) * sq, uint32_t( cnt_of( 0 ) ) * w16, waves );
     dma_publish();
     for ( int k = 0; k < K; ++k )
     {
         T *const cur = ( k & 1 ) ? buf1 : buf0;
         T *const nxt = ( k & 1 ) ? buf0 : buf1;
-        if ( k + 1 < K ) dma_copy16<BLOCK>( nxt, qhist + size_t( lo_of( k + 1 ) ) * sq, uint32_t( cnt_of( k + 1 ) ) * w16 );
+        if ( k + 1 < K ) dma_copy16( nxt, qhist + size_t( lo_of( k + 1 ) ) * sq, uint32_t( cnt_of( k + 1 ) ) * w16, waves );
         const int cnt = cnt_of( k );
         steps( cur, lo_of( k ), cnt - 1, 0 );
         dma_publish();
@@ -246,9 +246,9 @@ __device__ __forceinline__ void poly_ready_pipeline( T *lds, const T *qhist, uin
 
 // The same loop with one LDS buffer of C slices (tables too wide for two):
 // each chunk is copied, published, then traced.
-template <int BLOCK, typename T, typename STEPS>
+template <typename T, typename STEPS>
 __device__ __forceinline__ void poly_ready_direct( T *lds, const T *qhist, uint32_t sq, uint64_t n, uint32_t C,
-                                                   STEPS steps )
+                                                   uint32_t waves, STEPS steps )
 {
     const uint32_t w16 = sq * uint32_t( sizeof( T ) ) / 16u;
     for ( int mhi = int( n ) - 1; mhi >= 0; mhi -= int( C ) )
@@ -256,7 +256,7 @@ __device__ __forceinline__ void poly_ready_direct( T *lds, const T *qhist, uint3
         const int mlo = mhi - int( C ) + 1 > 0 ? mhi - int( C ) + 1 : 0;
         const int cnt = mhi - mlo + 1;
         __syncthreads();                            // the previous chunk's reads are done
-        dma_copy16<BLOCK>( lds, qhist + size_t( mlo ) * sq, uint32_t( cnt ) * w16 );
+        dma_copy16( lds, qhist + size_t( mlo ) * sq, uint32_t( cnt ) * w16, waves );
         dma_publish();
         steps( lds, mlo, cnt - 1, 0 );
     }

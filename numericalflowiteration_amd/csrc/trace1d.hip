@@ -105,17 +105,17 @@ __device__ __forceinline__ void write_partial( const trace1_params &p, const nod
 // ---- x-major layout (fast and FP32C rho kernels) ---------------------------
 struct xm_tile
 {
-    uint32_t xt, vb, xo, vr;   // x-tile, velocity block, lane's x offset and velocity row
-    bool lane_ok;              // the lane maps to an x node of the range
+    uint32_t xt, vb, xo, vr;   // x-tile, velocity block, the thread's x offset and velocity row
+    bool row_ok, lane_ok;      // the thread maps to a row of the tile; and to an x node of the range
 };
 
 __device__ __forceinline__ xm_tile make_tile( const trace1_params &p, uint32_t wg )
 {
     xm_tile t;
-    const uint32_t lane = threadIdx.x % WAVE;
     t.xt = wg % p.n_xt; t.vb = wg / p.n_xt;
-    t.xo = lane % p.xw; t.vr = lane / p.xw;
-    t.lane_ok = t.vr < p.vpw && t.xt * p.xw + t.xo < p.ix_count;
+    t.vr = threadIdx.x / p.xw; t.xo = threadIdx.x - t.vr * p.xw;
+    t.row_ok  = t.vr < p.rows;
+    t.lane_ok = t.row_ok && t.xt * p.xw + t.xo < p.ix_count;
     return t;
 }
 
@@ -125,14 +125,13 @@ struct xm_node
     bool active;
 };
 
-template <int WPB, int NPT>
+template <int NPT>
 __device__ __forceinline__ xm_node make_xm_node( const trace1_params &p, const xm_tile &t, int r )
 {
     xm_node id;
-    const uint32_t wave = threadIdx.x / WAVE;
-    id.vi = ( uint32_t( r ) * WPB + wave ) * p.vpw + t.vr;
+    id.vi = uint32_t( r ) * p.rows + t.vr;
     id.ix = t.lane_ok ? p.ix_first + t.xt * p.xw + t.xo : p.ix_first;
-    id.iu = t.vb * ( uint32_t( NPT * WPB ) * p.vpw ) + id.vi;
+    id.iu = t.vb * ( uint32_t( NPT ) * p.rows ) + id.vi;
     const uint64_t q = uint64_t( id.ix ) * p.Nu + id.iu;
     id.active = t.lane_ok && id.iu < p.Nu && q >= p.q_begin && q < p.q_end;
     return id;
@@ -141,20 +140,19 @@ __device__ __forceinline__ xm_node make_xm_node( const trace1_params &p, const x
 // f of the workgroup's nodes -> LDS -> one compensated sum per (x, group of
 // XM_GROUP consecutive velocities), summed in iu order, at partials[group*Nx + x].  `fbuf` may alias the
 // history chunk: the barrier below ends its use.
-template <int BLOCK, int NPT>
+template <int NPT>
 __device__ __forceinline__ void xm_reduce( const trace1_params &p, const xm_tile &t, const xm_node id[NPT],
                                            const double f[NPT], double *fbuf )
 {
-    constexpr uint32_t WPB = BLOCK / WAVE;
-    const uint32_t groups = ( uint32_t( NPT ) * WPB * p.vpw ) / XM_GROUP;
+    const uint32_t groups = ( uint32_t( NPT ) * p.rows ) / XM_GROUP;
     __syncthreads();
-    if ( t.vr < p.vpw )
+    if ( t.row_ok )
     {
         #pragma unroll
         for ( int r = 0; r < NPT; ++r ) fbuf[ id[r].vi * p.xw + t.xo ] = id[r].active ? f[r] : 0.0;
     }
     __syncthreads();
-    for ( uint32_t k = threadIdx.x; k < groups * p.xw; k += BLOCK )
+    for ( uint32_t k = threadIdx.x; k < groups * p.xw; k += blockDim.x )
     {
         const uint32_t xo = k % p.xw, gi = k / p.xw;
         const uint32_t xl = t.xt * p.xw + xo, gg = t.vb * groups + gi;
@@ -307,17 +305,16 @@ void trace1d_strict_kernel( trace1_params p )
 // two FMAs for Q0 + t (Q1 + t Q2), one FMA for the kick.  The tables are
 // copied from p.qhist into LDS by direct loads, double-buffered when p.pipe is
 // set (poly_ready_pipeline), else one buffer per chunk (poly_ready_direct).
-template <int BLOCK, int NPT, bool POW2>
+template <int NPT, bool POW2, int BLOCK>
 __device__ __forceinline__ void trace1d_poly_body( const trace1_params &p, uint32_t wg, double *lds )
 {
-    constexpr int WPB = BLOCK / WAVE;
     const xm_tile tile = make_tile( p, wg );
     xm_node id[NPT];
     double s[NPT], u[NPT];
     #pragma unroll
     for ( int r = 0; r < NPT; ++r )
     {
-        id[r] = make_xm_node<WPB,NPT>( p, tile, r );
+        id[r] = make_xm_node<NPT>( p, tile, r );
         s[r] = double( id[r].ix );
         u[r] = p.nu_min + id[r].iu*p.ndu + p.ndu/2;          // cuda_kernel.cu:44
     }
@@ -357,30 +354,35 @@ __device__ __forceinline__ void trace1d_poly_body( const trace1_params &p, uint3
             }
         }
     };
-    if ( p.pipe ) poly_ready_pipeline<BLOCK>( lds, p.qhist, sq, p.n, p.chunk, steps );
-    else          poly_ready_direct<BLOCK>( lds, p.qhist, sq, p.n, p.chunk, steps );
+    const uint32_t waves = BLOCK > 0 ? uint32_t( BLOCK / WAVE ) : blockDim.x / WAVE;
+    if ( p.pipe ) poly_ready_pipeline( lds, p.qhist, sq, p.n, p.chunk, waves, steps );
+    else          poly_ready_direct( lds, p.qhist, sq, p.n, p.chunk, waves, steps );
 
     double f[NPT];
     #pragma unroll
     for ( int r = 0; r < NPT; ++r ) f[r] = id[r].active ? f0_1d( p.f0, p.x_min + s[r]*p.dx, u[r] ) : 0.0;
-    xm_reduce<BLOCK,NPT>( p, tile, id, f, lds );
+    xm_reduce<NPT>( p, tile, id, f, lds );
 }
 
-template <int BLOCK, int NPT, bool POW2>
-__global__ __launch_bounds__( BLOCK )
+// BLOCK = 0: any workgroup size up to the limit (512 with four nodes a
+// thread); a full workgroup of 1024 threads gets its own instance, with the
+// wave count a constant in the copies
+constexpr int xm_max_block( int npt ) { return npt == 4 ? 512 : 1024; }
+
+template <int NPT, bool POW2, int BLOCK>
+__global__ __launch_bounds__( xm_max_block( NPT ) )
 void trace1d_poly_kernel( trace1_params p )
 {
     extern __shared__ double lds[];
-    trace1d_poly_body<BLOCK,NPT,POW2>( p, blockIdx.x, lds );
+    trace1d_poly_body<NPT,POW2,BLOCK>( p, blockIdx.x, lds );
 }
 
 // ---- FP32 compensated (order 4) --------------------------------------------
 // The FP32 kick-polynomial table: an 8-byte (Q0, Q1) and a 4-byte Q2 LDS
 // read per char-step.
-template <int BLOCK, int NPT, bool POW2>
+template <int NPT, bool POW2, int BLOCK>
 __device__ __forceinline__ void trace1d_fp32c_body( const trace1_params &p, uint32_t wg, float *ldsf )
 {
-    constexpr int WPB = BLOCK / WAVE;
     const xm_tile tile = make_tile( p, wg );
     xm_node id[NPT];
     float sh[NPT], sl[NPT], uh[NPT], ul[NPT];       // position (cells) + P0, velocity (cells per step) + W0
@@ -389,7 +391,7 @@ __device__ __forceinline__ void trace1d_fp32c_body( const trace1_params &p, uint
     #pragma unroll
     for ( int r = 0; r < NPT; ++r )
     {
-        id[r] = make_xm_node<WPB,NPT>( p, tile, r );
+        id[r] = make_xm_node<NPT>( p, tile, r );
         fp32c_start( fr, id[r].ix, cd * ( p.nu_min + id[r].iu*p.ndu + p.ndu/2 ), sh[r], sl[r], uh[r], ul[r] );
     }
 
@@ -432,8 +434,9 @@ __device__ __forceinline__ void trace1d_fp32c_body( const trace1_params &p, uint
             if ( seg == 0 && m == 0 ) { step( Q, 0.5f ); --m; Q -= sq; }
         }
     };
-    if ( p.pipe ) poly_ready_pipeline<BLOCK>( ldsf, p.qhist32, sq, p.n, p.chunk, steps );
-    else          poly_ready_direct<BLOCK>( ldsf, p.qhist32, sq, p.n, p.chunk, steps );
+    const uint32_t waves = BLOCK > 0 ? uint32_t( BLOCK / WAVE ) : blockDim.x / WAVE;
+    if ( p.pipe ) poly_ready_pipeline( ldsf, p.qhist32, sq, p.n, p.chunk, waves, steps );
+    else          poly_ready_direct( ldsf, p.qhist32, sq, p.n, p.chunk, waves, steps );
 
     double f[NPT];
     #pragma unroll
@@ -443,23 +446,23 @@ __device__ __forceinline__ void trace1d_fp32c_body( const trace1_params &p, uint
         const double u = fp32c_velocity( fr, uh[r], ul[r] ) / cd;
         f[r] = id[r].active ? f0_1d( p.f0, p.x_min + s*p.dx, u ) : 0.0;
     }
-    xm_reduce<BLOCK,NPT>( p, tile, id, f, reinterpret_cast<double*>( ldsf ) );
+    xm_reduce<NPT>( p, tile, id, f, reinterpret_cast<double*>( ldsf ) );
 }
 
-template <int BLOCK, int NPT, bool POW2>
-__global__ __launch_bounds__( BLOCK )
+template <int NPT, bool POW2, int BLOCK>
+__global__ __launch_bounds__( xm_max_block( NPT ) )
 void trace1d_fp32c_kernel( trace1_params p )
 {
     extern __shared__ float ldsf[];
-    trace1d_fp32c_body<BLOCK,NPT,POW2>( p, blockIdx.x, ldsf );
+    trace1d_fp32c_body<NPT,POW2,BLOCK>( p, blockIdx.x, ldsf );
 }
 
 // ---- batched sweep: one launch over the wave-tasks of many independent runs --
 // Workgroup b belongs to run wg_run[b]; its parameter block lives in device
 // memory (runs[r].p, with n filled in here) and its workgroup index within the
 // run is b - runs[r].wg_begin.  Runs past their own Nt skip the step.
-template <int BLOCK, int NPT, int VARIANT>
-__global__ __launch_bounds__( BLOCK )
+template <int NPT, int VARIANT>
+__global__ __launch_bounds__( xm_max_block( NPT ) )
 void trace1d_batch_kernel( const batch_run *__restrict__ runs, const uint32_t *__restrict__ wg_run, uint64_t n )
 {
     extern __shared__ double lds_b[];
@@ -471,11 +474,11 @@ void trace1d_batch_kernel( const batch_run *__restrict__ runs, const uint32_t *_
     const bool pow2 = ( p.Nx & ( p.Nx - 1 ) ) == 0;
     if ( VARIANT == TRACE_FP32C )
     {
-        if ( pow2 ) trace1d_fp32c_body<BLOCK,NPT,true>( p, wg, reinterpret_cast<float*>( lds_b ) );
-        else        trace1d_fp32c_body<BLOCK,NPT,false>( p, wg, reinterpret_cast<float*>( lds_b ) );
+        if ( pow2 ) trace1d_fp32c_body<NPT,true,0>( p, wg, reinterpret_cast<float*>( lds_b ) );
+        else        trace1d_fp32c_body<NPT,false,0>( p, wg, reinterpret_cast<float*>( lds_b ) );
     }
-    else if ( pow2 ) trace1d_poly_body<BLOCK,NPT,true>( p, wg, lds_b );
-    else        trace1d_poly_body<BLOCK,NPT,false>( p, wg, lds_b );
+    else if ( pow2 ) trace1d_poly_body<NPT,true,0>( p, wg, lds_b );
+    else        trace1d_poly_body<NPT,false,0>( p, wg, lds_b );
 }
 
 template <typename K>
@@ -492,32 +495,35 @@ hipError_t launch_kernel( K kernel, uint32_t grid, int block, size_t lds, const 
     return hipGetLastError();
 }
 
-template <int BLOCK, int NPT>
-hipError_t launch_fast_or_32( const trace1_params &p, int variant, uint32_t grid, size_t lds, hipStream_t st )
+template <int NPT, int BLOCK>
+hipError_t launch_xm_block( const trace1_params &p, int variant, uint32_t grid, uint32_t block, size_t lds, hipStream_t st )
 {
-    if ( p.mode == MODE_METRICS )
-        return launch_kernel( trace1d_fast_kernel<BLOCK,NPT,MODE_METRICS>, grid, BLOCK, lds, p, st );
+    const bool pow2 = ( p.Nx & ( p.Nx - 1 ) ) == 0;
     if ( variant == TRACE_FP32C )
-    {
-        if ( ( p.Nx & ( p.Nx - 1 ) ) == 0 )
-            return launch_kernel( trace1d_fp32c_kernel<BLOCK,NPT,true>, grid, BLOCK, lds, p, st );
-        return launch_kernel( trace1d_fp32c_kernel<BLOCK,NPT,false>, grid, BLOCK, lds, p, st );
-    }
-    if ( ( p.Nx & ( p.Nx - 1 ) ) == 0 )
-        return launch_kernel( trace1d_poly_kernel<BLOCK,NPT,true>, grid, BLOCK, lds, p, st );
-    return launch_kernel( trace1d_poly_kernel<BLOCK,NPT,false>, grid, BLOCK, lds, p, st );
+        return pow2 ? launch_kernel( trace1d_fp32c_kernel<NPT,true,BLOCK>,  grid, block, lds, p, st )
+                    : launch_kernel( trace1d_fp32c_kernel<NPT,false,BLOCK>, grid, block, lds, p, st );
+    return pow2 ? launch_kernel( trace1d_poly_kernel<NPT,true,BLOCK>,  grid, block, lds, p, st )
+                : launch_kernel( trace1d_poly_kernel<NPT,false,BLOCK>, grid, block, lds, p, st );
 }
 
-template <int BLOCK>
-hipError_t launch_npt( const trace1_params &p, int variant, int npt, uint32_t grid, size_t lds, hipStream_t st )
+hipError_t launch_xm( const trace1_params &p, int variant, int npt, uint32_t grid, uint32_t block, size_t lds, hipStream_t st )
 {
     switch ( npt )
     {
-    case 1: return launch_fast_or_32<BLOCK,1>( p, variant, grid, lds, st );
-    case 2: return launch_fast_or_32<BLOCK,2>( p, variant, grid, lds, st );
-    case 4: return launch_fast_or_32<BLOCK,4>( p, variant, grid, lds, st );
+    case 1: return block == 1024 ? launch_xm_block<1,1024>( p, variant, grid, block, lds, st )
+                                 : launch_xm_block<1,0>( p, variant, grid, block, lds, st );
+    case 2: return block == 1024 ? launch_xm_block<2,1024>( p, variant, grid, block, lds, st )
+                                 : launch_xm_block<2,0>( p, variant, grid, block, lds, st );
+    case 4: return launch_xm_block<4,0>( p, variant, grid, block, lds, st );
     default: return hipErrorInvalidValue;
     }
+}
+
+// the metrics launch: the wave-task cut, one node a thread
+template <int BLOCK>
+hipError_t launch_metrics( const trace1_params &p, uint32_t grid, size_t lds, hipStream_t st )
+{
+    return launch_kernel( trace1d_fast_kernel<BLOCK,1,MODE_METRICS>, grid, BLOCK, lds, p, st );
 }
 
 template <int ORDER, int MODE>
@@ -539,30 +545,17 @@ hipError_t launch_strict( const trace1_params &p, int block, uint32_t grid, size
     return launch_strict_mode<ORDER,MODE_RHO>( p, block, grid, lds, st );
 }
 
-template <int BLOCK, int NPT>
+template <int NPT>
 hipError_t launch_batch_npt( const batch_run *runs, const uint32_t *wg_run, uint32_t n_wg, uint64_t n,
-                             int variant, size_t lds, hipStream_t st )
+                             int variant, uint32_t block, size_t lds, hipStream_t st )
 {
     if ( variant == TRACE_FP32C )
-        hipLaunchKernelGGL( ( trace1d_batch_kernel<BLOCK,NPT,TRACE_FP32C> ), dim3( n_wg ), dim3( BLOCK ), lds, st,
+        hipLaunchKernelGGL( ( trace1d_batch_kernel<NPT,TRACE_FP32C> ), dim3( n_wg ), dim3( block ), lds, st,
                             runs, wg_run, n );
     else
-        hipLaunchKernelGGL( ( trace1d_batch_kernel<BLOCK,NPT,TRACE_FAST> ), dim3( n_wg ), dim3( BLOCK ), lds, st,
+        hipLaunchKernelGGL( ( trace1d_batch_kernel<NPT,TRACE_FAST> ), dim3( n_wg ), dim3( block ), lds, st,
                             runs, wg_run, n );
     return hipGetLastError();
-}
-
-template <int BLOCK>
-hipError_t launch_batch_block( const batch_run *runs, const uint32_t *wg_run, uint32_t n_wg, uint64_t n,
-                               int variant, int npt, size_t lds, hipStream_t st )
-{
-    switch ( npt )
-    {
-    case 1: return launch_batch_npt<BLOCK,1>( runs, wg_run, n_wg, n, variant, lds, st );
-    case 2: return launch_batch_npt<BLOCK,2>( runs, wg_run, n_wg, n, variant, lds, st );
-    case 4: return launch_batch_npt<BLOCK,4>( runs, wg_run, n_wg, n, variant, lds, st );
-    default: return hipErrorInvalidValue;
-    }
 }
 
 } // namespace
@@ -572,14 +565,13 @@ hipError_t launch_trace1d_batch( const batch_run *runs, const uint32_t *wg_run, 
 {
     if ( ( variant != TRACE_FAST && variant != TRACE_FP32C ) || n >= ( uint64_t( 1 ) << 31 ) ) return hipErrorInvalidValue;
     if ( n_wg == 0 ) return hipSuccess;
-    switch ( s.block )
+    const uint32_t block = uint32_t( s.block );
+    switch ( s.npt )
     {
-    case 64:   return launch_batch_block<64>  ( runs, wg_run, n_wg, n, variant, s.npt, lds, st );
-    case 128:  return launch_batch_block<128> ( runs, wg_run, n_wg, n, variant, s.npt, lds, st );
-    case 256:  return launch_batch_block<256> ( runs, wg_run, n_wg, n, variant, s.npt, lds, st );
-    case 512:  return launch_batch_block<512> ( runs, wg_run, n_wg, n, variant, s.npt, lds, st );
-    case 1024: return launch_batch_block<1024>( runs, wg_run, n_wg, n, variant, s.npt, lds, st );
-    default:   return hipErrorInvalidValue;
+    case 1: return launch_batch_npt<1>( runs, wg_run, n_wg, n, variant, block, lds, st );
+    case 2: return launch_batch_npt<2>( runs, wg_run, n_wg, n, variant, block, lds, st );
+    case 4: return launch_batch_npt<4>( runs, wg_run, n_wg, n, variant, block, lds, st );
+    default: return hipErrorInvalidValue;
     }
 }
 
@@ -613,12 +605,45 @@ static bool x_major( const trace1_params &p, int variant )
     return p.mode == MODE_RHO && variant != TRACE_STRICT;
 }
 
-void trace1d_xm_setup( trace1_params &p )
+// The tile of an x-major launch: xw x nodes by `rows` velocity rows a pass,
+// rows * npt whole summation groups, xw * rows threads (idle threads round the
+// workgroup up to whole waves).  The partial sums do not depend on it.
+//
+// spread = true (one-group workgroups of a single run: 1024 threads, one node
+// each): 16 rows, and the x axis cut into as many tiles as keep the grid
+// within one workgroup per CU (n_cu), down to 16 wide (one wave per SIMD) and
+// at most 64.  A run's step of few nodes is a chain of dependent steps, so
+// what counts is how many of them share a SIMD: the trace of 64 x 256 nodes at
+// n = 240 took 33.0 us in 16 workgroups of 16 waves and takes 24.2 in 64 of
+// 4; 128 x 512 at n = 160 30.6 -> 23.3; 100 x 515 at n = 160 (lanes of a
+// 64-wide tile no longer idle over 100 points either) 27.0 -> 19.9.
+// spread = false (a given block, batch launches): the tile count that leaves
+// the fewest lanes idle, the widest tile on ties.
+uint32_t trace1d_xm_setup( trace1_params &p, const launch_shape &s, bool spread, int n_cu )
 {
-    p.xw   = xm_xw( p.Nx );
-    p.vpw  = WAVE / p.xw;
-    p.n_xt = ( p.ix_count + p.xw - 1 ) / p.xw;
-    p.ppx  = xm_ppx( p.Nu );
+    p.ppx = xm_ppx( p.Nu );
+    const uint32_t nx = p.ix_count > 0 ? p.ix_count : 1;
+    const uint32_t k0 = ( nx + 63 ) / 64, k1 = ( nx + 15 ) / 16;
+    uint32_t k = k0;
+    if ( spread )
+    {
+        k = std::min( std::max( uint32_t( n_cu ) / p.ppx, k0 ), k1 );
+        p.xw = ( nx + k - 1 ) / k;
+        p.rows = XM_GROUP;
+    }
+    else
+    {
+        const uint32_t unit = XM_GROUP / std::min<uint32_t>( XM_GROUP, uint32_t( s.npt ) );
+        uint64_t best = 0;
+        for ( uint32_t c = k0; c <= k1; ++c )
+        {
+            const uint32_t xw = ( nx + c - 1 ) / c, rows = uint32_t( s.block ) / xw / unit * unit;
+            const uint64_t used = uint64_t( nx ) * rows * 65536u / c;      // ~ busy lanes per workgroup
+            if ( rows > 0 && used > best ) { best = used; p.xw = xw; p.rows = rows; }
+        }
+    }
+    p.n_xt = ( nx + p.xw - 1 ) / p.xw;
+    return ( p.xw * p.rows + WAVE - 1 ) / WAVE * WAVE;
 }
 
 // the FP64 and FP32C rho kernels read their tables from qhist / qhist32
@@ -643,7 +668,7 @@ uint32_t trace1d_grid( const trace1_params &p, int variant, const launch_shape &
 {
     if ( x_major( p, variant ) )
     {
-        const uint32_t vbw = uint32_t( s.block / WAVE ) * uint32_t( s.npt ) * p.vpw;
+        const uint32_t vbw = uint32_t( s.npt ) * p.rows;
         return p.n_xt * ( ( p.Nu + vbw - 1 ) / vbw );
     }
     const uint32_t tasks_per_block = uint32_t( s.block / WAVE ) * uint32_t( s.npt );
@@ -669,24 +694,27 @@ size_t trace1d_lds_bytes( const trace1_params &p, int variant, const launch_shap
     return hist > fbuf ? hist : fbuf;
 }
 
-hipError_t launch_trace1d( const trace1_params &p_in, int variant, const launch_shape &s, hipStream_t st )
+hipError_t launch_trace1d( const trace1_params &p_in, int variant, const launch_shape &s, int n_cu, hipStream_t st )
 {
     if ( !shape_built( variant, int( p_in.order ), s ) || p_in.n >= ( uint64_t( 1 ) << 31 ) ) return hipErrorInvalidValue;
     trace1_params p = p_in;
-    if ( x_major( p, variant ) )
+    const bool xm = x_major( p, variant );
+    uint32_t block = uint32_t( s.block );
+    if ( xm )
     {
         if ( !shape_groups( s ) ) return hipErrorInvalidValue;
-        trace1d_xm_setup( p );
         if ( p.ix_count == 0 ) return hipSuccess;
+        // the x-major rho kernels copy the kick-polynomial tables of the history
+        if ( !poly_ready( p, variant ) ) return hipErrorInvalidValue;
+        block = trace1d_xm_setup( p, s, s.block == 1024 && s.npt == 1, n_cu );     // one-group workgroups narrow to fill the chip
     }
     else if ( p.n_tasks == 0 ) return hipSuccess;
-    // the x-major rho kernels copy the kick-polynomial tables of the history
-    if ( x_major( p, variant ) && !poly_ready( p, variant ) ) return hipErrorInvalidValue;
     const uint32_t grid = trace1d_grid( p, variant, s );
     bool pipe = false;
     p.chunk = trace1d_chunk( p, variant, s, 160 * 1024, &pipe );
     p.pipe = pipe ? 1u : 0u;
     const size_t lds = trace1d_lds_bytes( p, variant, s );
+    if ( xm ) return launch_xm( p, variant, s.npt, grid, block, lds, st );
 
     if ( variant == TRACE_STRICT )
     {
@@ -701,13 +729,10 @@ hipError_t launch_trace1d( const trace1_params &p_in, int variant, const launch_
         default: return hipErrorInvalidValue;
         }
     }
+    if ( s.npt != 1 ) return hipErrorInvalidValue;
     switch ( s.block )
     {
-    case 64:   return launch_npt<64>  ( p, variant, s.npt, grid, lds, st );
-    case 128:  return launch_npt<128> ( p, variant, s.npt, grid, lds, st );
-    case 256:  return launch_npt<256> ( p, variant, s.npt, grid, lds, st );
-    case 512:  return launch_npt<512> ( p, variant, s.npt, grid, lds, st );
-    case 1024: return launch_npt<1024>( p, variant, s.npt, grid, lds, st );
+    case 256:  return launch_metrics<256>( p, grid, lds, st );
     default:   return hipErrorInvalidValue;
     }
 }
