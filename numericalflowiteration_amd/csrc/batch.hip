@@ -93,6 +93,32 @@ void bfree_all( nufi_batch *b )
     if ( b->stream ) (void)hipStreamDestroy( b->stream );
 }
 
+// LDS of a batch workgroup: a third of a CU's, so that three workgroups of 512
+// threads share it.  Their waves sit at different points of their chunks, and
+// the more of them a SIMD holds the better VALU and LDS overlap: 512 runs to
+// T = 5 at 512 x 4 took 78.0 ms with two workgroups of 64 KiB, 76.2 with two of
+// 80 KiB, 70.2 with three of 52 KiB and 71.6 with four of 40 KiB (FP32C; FP64
+// 74.8, 73.0, 68.5, 72.2).  Grids whose two table rows do not fit it take 64 KiB.
+constexpr size_t BATCH_LDS = 52 * 1024, BATCH_LDS_MAX = 64 * 1024;
+
+size_t batch_lds( const nufi_batch *b )
+{
+    const size_t elem = b->variant == TRACE_FP32C ? sizeof(float) : sizeof(double);
+    return 2 * size_t( b->max_sq ) * elem <= BATCH_LDS ? BATCH_LDS : BATCH_LDS_MAX;
+}
+
+// The shape of a new batch (the autotuner refines it).  Four nodes a thread
+// trace four times the steps per copied slice and barrier; with few nodes the
+// workgroups then leave CUs idle.  T = 10, FP32C / FP64: 0.82M nodes 512 x 4
+// 9.0 / 9.4 ms, 512 x 2 9.6 / 11.4, 1024 x 1 11.5 / 13.8; 0.28M nodes 6.6 /
+// 7.0, 5.8 / 6.5, 6.6 / 7.4; 0.02M nodes 5.5 / 5.3, 3.9 / 3.9, 3.7 / 3.8.
+launch_shape batch_default_shape( uint64_t nodes, int chunk )
+{
+    if ( nodes >= 600000 ) return launch_shape { 512, 4, chunk };
+    if ( nodes >= 150000 ) return launch_shape { 512, 2, chunk };
+    return launch_shape { 1024, 1, chunk };
+}
+
 // (Re)build the workgroup table and the run descriptors for the current shape.
 int apply_shape( nufi_batch *b, const launch_shape &s )
 {
@@ -102,6 +128,7 @@ int apply_shape( nufi_batch *b, const launch_shape &s )
     // per run: the table chunk (bounded by the register prefetch) and its LDS,
     // or the x-major f buffer of the workgroup, whichever is larger
     size_t lds = size_t( s.block ) * size_t( s.npt ) * sizeof(double);
+    const size_t lds_cap = batch_lds( b );
     std::vector<uint32_t> wg_run;
     for ( uint64_t r = 0; r < b->n_runs; ++r )
     {
@@ -109,7 +136,7 @@ int apply_shape( nufi_batch *b, const launch_shape &s )
         trace1_params q = h.p;
         q.n = h.Nt;                                    // the chunk bound of the longest step
         bool pipe = false;
-        h.p.chunk = trace1d_chunk( q, b->variant, s, 65536, &pipe );
+        h.p.chunk = trace1d_chunk( q, b->variant, s, lds_cap, &pipe );
         h.p.pipe = pipe ? 1u : 0u;
         lds = std::max( lds, ( pipe ? 2 : 1 ) * size_t( h.p.chunk ) * b->sq[r] * elem );
         (void)trace1d_xm_setup( h.p, s, false, 0 );
@@ -117,7 +144,7 @@ int apply_shape( nufi_batch *b, const launch_shape &s )
         h.n_wg = trace1d_grid( h.p, b->variant, s );
         wg_run.insert( wg_run.end(), h.n_wg, uint32_t( r ) );
     }
-    if ( lds > 65536 ) return bfail( b, NUFI_ERR_UNSUPPORTED, "batch: launch shape needs more than 64 KiB of LDS" );
+    if ( lds > BATCH_LDS_MAX ) return bfail( b, NUFI_ERR_UNSUPPORTED, "batch: launch shape needs more than 64 KiB of LDS" );
     if ( wg_run.size() >= ( size_t( 1 ) << 31 ) ) return bfail( b, NUFI_ERR_RANGE, "batch: too many workgroups" );
     if ( wg_run.size() > b->d_wg_cap )
     {
@@ -277,8 +304,10 @@ int nufi_batch_create( const nufi_config *confs, uint64_t n_runs, int order, int
     { bhip( b, he, "batch table upload" ); return bail( NUFI_ERR_DEVICE ); }
 
     const size_t elem = b->variant == TRACE_FP32C ? sizeof(float) : sizeof(double);
-    const int chunk = int( std::max<size_t>( 1, std::min<size_t>( 64, 65536 / ( size_t( b->max_sq ) * elem ) ) ) );
-    if ( ( rc = apply_shape( b, launch_shape { 1024, 1, chunk } ) ) ) return bail( rc );
+    uint64_t nodes = 0;
+    for ( const nufi_config &c : b->confs ) nodes += c.Nx * c.Nu;
+    const int chunk = int( std::max<size_t>( 1, std::min<size_t>( 64, batch_lds( b ) / ( size_t( b->max_sq ) * elem ) ) ) );
+    if ( ( rc = apply_shape( b, batch_default_shape( nodes, chunk ) ) ) ) return bail( rc );
     *out = b;
     return NUFI_OK;
 }
@@ -379,7 +408,7 @@ int nufi_batch_autotune( nufi_batch *b, uint64_t n_probe, int repeats, int *bloc
     BHIP( b, hipSetDevice( b->device ) );
     BHIP( b, hipStreamSynchronize( b->stream ) );
     const size_t elem = b->variant == TRACE_FP32C ? sizeof(float) : sizeof(double);
-    const int cmax = int( std::max<size_t>( 1, std::min<size_t>( 64, 65536 / ( size_t( b->max_sq ) * elem ) ) ) );
+    const int cmax = int( std::max<size_t>( 1, std::min<size_t>( 64, batch_lds( b ) / ( size_t( b->max_sq ) * elem ) ) ) );
     const launch_shape saved = b->shape;
     hipEvent_t e0, e1;
     BHIP( b, hipEventCreate( &e0 ) );
