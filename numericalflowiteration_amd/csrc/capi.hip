@@ -41,6 +41,7 @@ struct nufi_ctx
     uint32_t wpx = 0;          // wave-task partials per spatial point (strict 1D, 3D)
     uint32_t ppx = 0;          // x-major partials per spatial point (fast; 1D FP32C)
     uint32_t vgroup = 0;       // 3D x-major: velocities per partial
+    zcell_plan zc {};          // 3D fast FP64 (rho and metrics): the z-cell kernel's layout, zc.ok where it runs
     int field_ok = 0;          // 1: one-workgroup field solve; 2: the multi-workgroup one; 0: none
     double2 *lw0 = nullptr, *lw1 = nullptr;   // multi-workgroup solve: two complex buffers
     double *lpart = nullptr;                  // and its energy partials
@@ -130,7 +131,7 @@ void free_all( nufi_ctx *c )
     void *ptrs[] = { c->hist, c->dhist, c->qhist, c->qhist32, c->hist32, c->partials, c->rho, c->energies,
                      c->values, c->scratch_slice, c->metrics, c->mpartials, c->energy_tmp,
                      c->rho_hist, c->lambda, c->gvec, c->grad_part, c->grad, c->tw_x, c->tw_y, c->tw_z,
-                     c->mult_step, c->mult_pois, c->mult_fit, c->ewt, c->samp, c->lw0, c->lw1, c->lpart };
+                     c->mult_step, c->mult_pois, c->mult_fit, c->ewt, c->samp, c->lw0, c->lw1, c->lpart, c->zc.marks };
     if ( c->run_graph ) (void)hipGraphExecDestroy( c->run_graph );
     c->run_graph = nullptr;
     for ( void *p : ptrs ) if ( p ) (void)hipFree( p );
@@ -265,8 +266,8 @@ void default_shape( nufi_ctx *c )
         const size_t per = size_t( c->st ) * elem;
         int chunk = int( std::min<size_t>( c->lds_cap, 64 * 1024 ) / per );
         chunk = std::max( 1, std::min( chunk, 1 ) );
-        // the autotuner's picks on 16^3 x 32^3 (two 1-slice buffers each); eight
-        // FP64 nodes a lane trace twice the node-steps per slice barrier of four
+        // FP32C: the autotuner's pick on 16^3 x 32^3 (two 1-slice buffers); FP64:
+        // the z-cell kernel has one shape (512 x 8), its window kernel takes four for eight
         if ( c->variant == TRACE_STRICT ) c->shape = launch_shape { 256, 1, chunk };
         else if ( c->variant == TRACE_FP32C ) c->shape = launch_shape { 512, 4, 1 };
         else c->shape = launch_shape { 512, 8, chunk };
@@ -331,7 +332,7 @@ int launch_trace( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_end, uin
         p.Nu = uint32_t( c->conf.Nu ); p.Nv = uint32_t( c->conf.Nv ); p.Nw = uint32_t( c->conf.Nw );
         p.sy = c->sy; p.sz = c->sz; p.st = c->st; p.st32 = c->st32; p.wpx = c->wpx;
         p.l_first = uint32_t( l0 ); p.n_tasks = uint32_t( tasks );
-        p.n_count = uint32_t( l1 - l0 + 1 ); p.vgroup = c->vgroup; p.ppx = c->ppx;
+        p.n_count = uint32_t( l1 - l0 + 1 ); p.vgroup = c->vgroup; p.ppx = c->ppx; p.zc = c->zc;
         p.order = uint32_t( c->order );
         fill_trace3_geometry( p, c->conf );
         e = launch_trace3d( p, c->variant, c->shape, c->stream );
@@ -508,6 +509,8 @@ int nufi_create( const nufi_config *conf, const nufi_config *conf_metrics, int o
     {
         c->vgroup = xm3_vgroup( c->n_space, c->n_vel );
         c->ppx = uint32_t( ( c->n_vel + c->vgroup - 1 ) / c->vgroup );
+        c->zc = plan_zcell( *conf );
+        if ( c->zc.ok ) c->ppx = c->zc.ppx;
     }
     c->field_ok = field_supported( c->dim, uint32_t( conf->Nx ), c->dim == 3 ? uint32_t( conf->Ny ) : 1u,
                                    c->dim == 3 ? uint32_t( conf->Nz ) : 1u );
@@ -543,7 +546,9 @@ int nufi_create( const nufi_config *conf, const nufi_config *conf_metrics, int o
     else { c->m_space = c->n_space; c->m_vel = c->n_vel; }
     c->m_nodes = c->m_space * c->m_vel;
     c->m_wpx = uint32_t( ( c->m_vel + 63 ) / 64 );
-    if ( ( rc = dev_alloc( c, &c->mpartials, 4 * c->m_space * c->m_wpx, "metric partials" ) ) ) return bail( rc );
+    if ( c->zc.ok && ( rc = dev_alloc( c, &c->zc.marks, zcell_workgroups( *conf, c->zc, nullptr ), "window marks" ) ) ) return bail( rc );
+    const size_t m_waves = std::max<size_t>( c->m_space * c->m_wpx, c->zc.ok ? zcell_metric_waves( *conf, c->zc ) : 0 );
+    if ( ( rc = dev_alloc( c, &c->mpartials, 4 * m_waves, "metric partials" ) ) ) return bail( rc );
     if ( c->field_ok && ( rc = build_tables( c ) ) ) return bail( rc );
     c->host_rho.assign( c->n_space, 0.0 );
     default_shape( c );
@@ -681,7 +686,14 @@ int nufi_compute_metrics( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_
             p.sy = c->sy; p.sz = c->sz; p.st = c->st; p.wpx = c->m_wpx;
             p.l_first = uint32_t( l0 ); p.n_tasks = uint32_t( tasks ); p.order = uint32_t( c->order );
             fill_trace3_geometry( p, g );
-            e = launch_trace3d( p, variant, launch_shape { 256, 1, 1 }, c->stream );
+            if ( variant == TRACE_FAST && c->zc.ok )
+            {
+                uint32_t waves = 0;
+                p.n_count = uint32_t( l1 - l0 + 1 ); p.zc = c->zc;
+                e = launch_trace3d_zcell( p, &waves, c->stream );
+                tasks = waves;
+            }
+            else e = launch_trace3d( p, variant, launch_shape { 256, 1, 1 }, c->stream );
         }
         if ( e != hipSuccess ) return hip_fail( c, e, "metrics trace launch" );
     }

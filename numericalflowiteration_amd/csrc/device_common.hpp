@@ -49,7 +49,7 @@ __device__ inline double f0_1d( const nufi_f0 &p, double x, double u )
     }
 }
 
-__device__ inline double f0_3d( const nufi_f0 &p, double x, double y, double z,
+__device__ __forceinline__ double f0_3d( const nufi_f0 &p, double x, double y, double z,
                                 double u, double v, double w )
 {
 #pragma clang fp contract(off)
@@ -124,6 +124,13 @@ __device__ __forceinline__ double wave_sum( double v )
     for ( int off = WAVE/2; off > 0; off >>= 1 )
         v += __shfl_xor( v, off );
     return v;
+}
+
+// One direct global->LDS load: lane l's 16 bytes at g to LDS byte m0 + 16 l
+// (m0 uniform; see dma_copy16).
+__device__ __forceinline__ void dma_issue16( const char *g, uint32_t m0 )
+{
+    asm volatile( "s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"( g ), "{m0}"( m0 ) : "memory" );
 }
 
 // Direct global->LDS copy of n16 16-byte words (gfx950 global_load_lds_dwordx4)

@@ -97,6 +97,45 @@ inline uint32_t xm3_vgroup( uint64_t n_space, uint64_t n_vel )
     while ( g > 16 && tiles * ( ( n_vel + g - 1 ) / g ) < 8192 ) g /= 2;
     return g;
 }
+// The z-cell trace (trace3d_zcell.hip).  Velocity group g of w index iw: the
+// (u, v) indices g*vg .. g*vg+vg-1 (u innermost); its partial sum is
+// partials[(iw*ngw + g)*n_space + l].
+constexpr uint32_t ZCELL_PAIR2 = 48 * 1024, ZCELL_MAX = 4, ZCELL_MARKS = 1u << 16;
+struct zcell_consts          // per axis: points, their inverse, drift in cells per unit velocity, kick constants
+{
+    double N[3], iN[3], cd[3], kick[3], kickh[3];
+};
+struct zcell_plan
+{
+    bool ok;
+    uint32_t nzc;            // z-cells of a workgroup's window
+    uint32_t szp;            // doubles a staged coefficient plane takes (one plane and its alignment)
+    uint32_t vg, ngw, ppx;   // velocities per group, groups per w, partials per point
+    uint32_t tw, gpw, tiles, ngb, z_first;     // per launch: points and groups of a workgroup, tiles a plane,
+                                               // group blocks a w, first z plane
+    uint32_t inv_nx;         // ceil(2^20 / Nx)
+    uint32_t *marks;         // per workgroup: 1 where the window did not hold its nodes
+    zcell_consts k;
+};
+inline size_t zcell_lds( uint32_t nzc, uint32_t cols, uint32_t szp )
+{
+    return ZCELL_PAIR2 + 2ull * nzc * cols * 16u + 2ull * ( nzc + 3 ) * szp * 8u + 48u;
+}
+// Points (tw) by groups (gpw) of a workgroup of at most 512 threads for a
+// plane of P points and ngw groups: the busiest split, the widest tile on ties;
+// returns the share of a workgroup's lanes that trace.
+inline double zcell_tile( uint32_t P, uint32_t ngw, uint32_t *tw, uint32_t *gpw )
+{
+    constexpr uint32_t block = 512;
+    double best = 0;
+    for ( uint32_t c = ( P + block - 1 ) / block; c <= ( P + 15 ) / 16; ++c )
+    {
+        const uint32_t w = ( P + c - 1 ) / c, g = std::min( ngw, block / w ), nb = ( ngw + g - 1 ) / g;
+        const double use = double( P ) * ngw / ( double( c ) * nb * block );
+        if ( use > best ) { best = use; *tw = w; *gpw = ( ngw + nb - 1 ) / nb; }
+    }
+    return best;
+}
 struct trace3_params
 {
     const double *hist;      // coefficient slices (FP64), stride st
@@ -121,6 +160,7 @@ struct trace3_params
     double u_min, v_min, w_min, du, dv, dw, dt;
     double kick72[3], kick72h[3]; // fast FP64: -dt d_inv / 72 per axis (72-scaled gradient), and half of it
     float f32_p0[3], f32_w0[3];   // FP32C: offsets of the position and velocity hi parts per axis
+    zcell_plan zc;                // fast FP64: the z-cell kernel's layout (zc.ok), else the window kernel
     nufi_f0 f0;
 };
 
@@ -195,6 +235,14 @@ struct launch_shape
 // Launchers (trace1d.hip / trace3d.hip).  Return hipSuccess or the error.
 hipError_t launch_trace1d( const trace1_params &p, int variant, const launch_shape &s, int n_cu, hipStream_t st );
 hipError_t launch_trace3d( const trace3_params &p, int variant, const launch_shape &s, hipStream_t st );
+// The z-cell kernel for grids whose window fits the LDS (ok = false
+// otherwise): its groups depend on the grid alone.  *tasks: metrics partials written.
+zcell_plan plan_zcell( const nufi_config &g );
+// waves of a whole-grid metrics launch (its partials are four reals a wave)
+size_t zcell_metric_waves( const nufi_config &g, const zcell_plan &z );
+// workgroups (and their waves) of a whole-grid launch, at most ZCELL_MARKS; a mark each
+size_t zcell_workgroups( const nufi_config &g, const zcell_plan &z, uint32_t *waves );
+hipError_t launch_trace3d_zcell( const trace3_params &p, uint32_t *tasks, hipStream_t st );
 size_t trace1d_slice_elems( const trace1_params &p, int variant );
 hipError_t launch_trace1d_batch( const batch_run *runs, const uint32_t *wg_run, uint32_t n_wg, uint64_t n,
                                  int variant, const launch_shape &s, size_t lds, hipStream_t st );

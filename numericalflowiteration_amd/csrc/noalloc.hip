@@ -25,9 +25,11 @@ namespace
 
 constexpr size_t SCRATCH_DOUBLES = NUFI_NOALLOC_SCRATCH_BYTES / sizeof(double);
 static __device__ __align__( 256 ) double scratch[SCRATCH_DOUBLES];
+static __device__ uint32_t marks[nufi_impl::ZCELL_MARKS];          // the z-cell trace's window marks
 
 constexpr int MAX_DEVICES = 64;
 double *g_scratch[MAX_DEVICES] = {};
+uint32_t *g_marks[MAX_DEVICES] = {};
 std::mutex g_scratch_mu;
 
 int fail( int code, const std::string &msg )
@@ -36,8 +38,8 @@ int fail( int code, const std::string &msg )
     return code;
 }
 
-// The current device's copy of `scratch` (looked up once per device).
-int device_scratch( double **out )
+// The current device's copies of `scratch` and `marks` (looked up once per device).
+int device_scratch( double **out, uint32_t **out_marks )
 {
     int dev = 0;
     hipError_t e = hipGetDevice( &dev );
@@ -50,9 +52,15 @@ int device_scratch( double **out )
         e = hipGetSymbolAddress( &p, HIP_SYMBOL( scratch ) );
         if ( e != hipSuccess || p == nullptr )
             return fail( NUFI_ERR_DEVICE, std::string( "rho3d_noalloc: hipGetSymbolAddress: " ) + hipGetErrorString( e ) );
+        void *q = nullptr;
+        e = hipGetSymbolAddress( &q, HIP_SYMBOL( marks ) );
+        if ( e != hipSuccess || q == nullptr )
+            return fail( NUFI_ERR_DEVICE, std::string( "rho3d_noalloc: hipGetSymbolAddress: " ) + hipGetErrorString( e ) );
         g_scratch[dev] = static_cast<double*>( p );
+        g_marks[dev] = static_cast<uint32_t*>( q );
     }
     *out = g_scratch[dev];
+    *out_marks = g_marks[dev];
     return NUFI_OK;
 }
 
@@ -71,9 +79,10 @@ extern "C" int nufi_rho3d_noalloc( const nufi_config *conf, uint64_t n, const do
     const uint64_t sy = conf->Nx + order - 1, sz = sy * ( conf->Ny + order - 1 ), st = sz * ( conf->Nz + order - 1 );
     const uint64_t n_space = conf->Nx * conf->Ny * conf->Nz, n_vel = conf->Nu * conf->Nv * conf->Nw;
     const uint32_t vgroup = xm3_vgroup( n_space, n_vel );
-    const uint64_t ppx = ( n_vel + vgroup - 1 ) / vgroup;
-    if ( ppx * n_space > SCRATCH_DOUBLES )
-        return fail( NUFI_ERR_UNSUPPORTED, "rho3d_noalloc: this grid needs " + std::to_string( ppx * n_space * 8 ) +
+    const zcell_plan zc = plan_zcell( *conf );
+    const uint64_t ppw = ( n_vel + vgroup - 1 ) / vgroup, ppx = zc.ok ? zc.ppx : ppw;
+    if ( std::max( ppw, ppx ) * n_space > SCRATCH_DOUBLES )
+        return fail( NUFI_ERR_UNSUPPORTED, "rho3d_noalloc: this grid needs " + std::to_string( std::max( ppw, ppx ) * n_space * 8 ) +
                                            " bytes of partial sums, above the " +
                                            std::to_string( NUFI_NOALLOC_SCRATCH_BYTES ) + "-byte scratch array" );
     if ( st * sizeof(double) > 160 * 1024 )
@@ -91,7 +100,8 @@ extern "C" int nufi_rho3d_noalloc( const nufi_config *conf, uint64_t n, const do
             return fail( NUFI_ERR_INVALID, "rho3d_noalloc: the history must hold n slices and one more real" );
     }
     double *part = nullptr;
-    int rc = device_scratch( &part );
+    uint32_t *mk = nullptr;
+    int rc = device_scratch( &part, &mk );
     if ( rc ) return rc;
 
     trace3_params p {};
@@ -103,11 +113,11 @@ extern "C" int nufi_rho3d_noalloc( const nufi_config *conf, uint64_t n, const do
     p.sy = uint32_t( sy ); p.sz = uint32_t( sz ); p.st = uint32_t( st ); p.st32 = uint32_t( ( st + 3 ) & ~uint64_t( 3 ) );
     p.wpx = uint32_t( wpx );
     p.l_first = 0; p.n_tasks = uint32_t( n_space * wpx ); p.n_count = uint32_t( n_space );
-    p.vgroup = vgroup; p.ppx = uint32_t( ppx );
+    p.vgroup = vgroup; p.ppx = uint32_t( ppx ); p.zc = zc; p.zc.marks = mk;
     p.order = order;
     fill_trace3_geometry( p, *conf );
     const hipStream_t s = static_cast<hipStream_t>( stream );
-    hipError_t e = launch_trace3d( p, TRACE_FAST, launch_shape { 512, 4, 1 }, s );
+    hipError_t e = launch_trace3d( p, TRACE_FAST, launch_shape { 512, zc.ok ? 8 : 4, 1 }, s );
     if ( e != hipSuccess ) return fail( NUFI_ERR_DEVICE, std::string( "rho3d_noalloc: trace launch: " ) + hipGetErrorString( e ) );
     e = launch_reduce_partials( part, uint32_t( ppx ), -( conf->du * conf->dv * conf->dw ), 0, uint32_t( n_space ),
                                 uint32_t( n_space ), rho_dev, s );
