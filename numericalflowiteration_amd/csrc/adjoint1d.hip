@@ -51,7 +51,8 @@ __device__ inline void f0_grad_1d( const nufi_f0 &p, double x, double u, double 
     {
     case NUFI_F0_LANDAU_1D:
     {
-        const double c = cos( p.k*x ), s = sin( p.k*x );
+        double c, s;
+        sincos( p.k*x, &s, &c );
         fx = kInvSqrt2Pi * ( -p.alpha * p.k * s ) * e;
         fu = kInvSqrt2Pi * ( 1.0 + p.alpha*c ) * e * ( -u );
         if ( npar > 0 ) fa[0] = kInvSqrt2Pi * c * e;
@@ -59,7 +60,8 @@ __device__ inline void f0_grad_1d( const nufi_f0 &p, double x, double u, double 
     }
     case NUFI_F0_TWOSTREAM_1D:
     {
-        const double c = cos( p.k*x ), s = sin( p.k*x );
+        double c, s;
+        sincos( p.k*x, &s, &c );
         fx = kInvSqrt2Pi * ( -p.alpha * p.k * s ) * e * u*u;
         fu = kInvSqrt2Pi * ( 1.0 + p.alpha*c ) * e * u * ( 2.0 - u*u );
         if ( npar > 0 ) fa[0] = kInvSqrt2Pi * c * e * u*u;
@@ -73,7 +75,8 @@ __device__ inline void f0_grad_1d( const nufi_f0 &p, double x, double u, double 
         {
             if ( m > p.n_modes ) continue;
             const double km = p.k * m;
-            const double c = cos( km * x ), s = sin( km * x );
+            double c, s;
+            sincos( km * x, &s, &c );
             sm += p.a[m-1] * c;
             dsm -= p.a[m-1] * km * s;
             if ( m <= npar ) fa[m-1] = kInvSqrt2Pi * c * e;
@@ -89,215 +92,316 @@ __device__ inline void f0_grad_1d( const nufi_f0 &p, double x, double u, double 
     }
 }
 
-template <int BLOCK, bool POW2>
-__global__ __launch_bounds__( BLOCK )
-void adjoint1d_kernel( adjoint1_params p )
+// One node's state and its adjoint in each arithmetic: down() takes the forward
+// steps of slices mlo+hi .. mlo (tables at Q, sq elements each), locate() gives
+// the cell (in [-1, Nx]; POW2: in [0, Nx)) and t the forward step used at the
+// present position, undo() takes a step back (h = 1, or 1/2 on slice 0) and
+// returns pbar, the adjoint of the kick polynomial's value; with POW2 the
+// caller re-wraps behind every slice m with poly_wrap_due(m).
+template <bool POW2>
+struct adjoint_fp64
 {
-    extern __shared__ double lds[];
-    double *Ql  = lds;                                   // chunk of kick-polynomial slices
-    double *lam = lds + size_t( p.chunk ) * p.stride_q;  // chunk of folded slice adjoints
-    constexpr int WPB = BLOCK / WAVE;
-    const uint32_t lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-    const uint32_t g = blockIdx.x * WPB + wave;
-    const bool task = g < p.n_tasks;
-    const uint32_t ix = task ? g / p.wpx : 0, j = task ? g % p.wpx : 0;
-    const uint32_t iu = j * WAVE + lane;
-    const bool active = task && iu < p.Nu;
+    using table = double;
+    double cd, kick, Nxd, invNx, s, u, sbar, pb;          // pb: kick times the adjoint of u
+    int mask;
+    uint32_t q2;
 
-    const int Nx = int( p.Nx ), mask = Nx - 1;
-    const double Nxd = p.Nx, invNx = 1.0 / Nxd;
-    const double cd = p.dt * p.dx_inv, kick = -0.5 * p.dt * p.dx_inv;
-    const uint32_t sq = p.stride_q, q2 = p.q2_off;
-
-    double s = double( ix );
-    double u = p.u_min + iu*p.du + p.du/2;
-
-    // forward: slices n-1 .. 0, the step of trace1d_poly_body
-    for ( int64_t mhi = int64_t( p.n ) - 1; mhi >= 0; mhi -= p.chunk )
+    __device__ __forceinline__ static const double *tables( const adjoint1_params &p ) { return p.qhist; }
+    __device__ __forceinline__ void start( const adjoint1_params &p, uint32_t ix, uint32_t iu )
     {
-        const int64_t mlo = mhi - int64_t( p.chunk ) + 1 > 0 ? mhi - int64_t( p.chunk ) + 1 : 0;
-        const int cnt = int( mhi - mlo + 1 );
-        __syncthreads();
-        dma_copy16<BLOCK>( Ql, p.qhist + size_t( mlo ) * sq, uint32_t( cnt ) * sq / 2u );
-        dma_publish();
-        for ( int jj = cnt - 1; jj >= 0; )          // segments between re-wrap points
+        Nxd = p.Nx; invNx = 1.0 / Nxd; cd = p.dt * p.dx_inv; kick = -0.5 * p.dt * p.dx_inv;
+        mask = int( p.Nx ) - 1; q2 = p.q2_off;
+        s = double( ix );
+        u = p.u_min + iu*p.du + p.du/2;
+    }
+    __device__ __forceinline__ void down( const double *Q, uint32_t sq, int mlo, int hi )
+    {
+        for ( int jj = hi; jj >= 0; )          // segments between re-wrap points
         {
             if ( POW2 && poly_wrap_due( mlo + jj ) ) rewrap( s, Nxd, invNx );
-            const int jstop = POW2 ? int( poly_segment_end( mlo + jj, mlo ) - mlo ) : -1;
-            for ( ; jj > jstop; --jj )
-                poly_step<POW2>( s, u, Ql + jj * sq, Ql + jj * sq + q2, cd, ( mlo + jj == 0 ) ? 0.5 * kick : kick, mask,
-                                 Nxd, invNx );
+            const int jstop = POW2 ? int( poly_segment_end( mlo + jj, mlo ) ) - mlo : -1;
+            const int half = mlo == 0 && jstop < 0 ? 1 : 0;          // slice 0, the last of its segment
+            const double *R = Q + jj * sq;
+            #pragma unroll 4
+            for ( ; jj >= jstop + 1 + half; --jj, R -= sq ) poly_step<POW2>( s, u, R, R + q2, cd, kick, mask, Nxd, invNx );
+            if ( half ) { poly_step<POW2>( s, u, Q, Q + q2, cd, 0.5 * kick, mask, Nxd, invNx ); --jj; }
         }
     }
-
-    // seed at the foot
-    const double fbar = active ? -p.du * p.g[ix] : 0.0;
-    double fx, fu, fa[NUFI_MAX_MODES];
-    f0_grad_1d( p.f0, p.x_min + s*p.dx, u, fx, fu, fa, p.npar );
-    double sbar = fbar * fx * p.dx;     // d/ds = dx d/dx
-    double ubar = fbar * fu;
-    #pragma unroll
-    for ( int m = 0; m < NUFI_MAX_MODES; ++m )          // npar is uniform: the branch is too
+    __device__ __forceinline__ double foot_x( const adjoint1_params &p ) const { return p.x_min + s*p.dx; }
+    __device__ __forceinline__ double foot_u() const { return u; }
+    __device__ __forceinline__ void seed( const adjoint1_params &p, double fbar, double fx, double fu )
     {
-        if ( m >= int( p.npar ) ) continue;
-        const csum v = wave_csum( csum { fbar * fa[m], 0.0 } );
-        if ( task && lane == 0 ) p.grad_part[ size_t( g ) * NUFI_MAX_MODES + m ] += v.s + v.c;
+        sbar = fbar * fx * p.dx;               // d/ds = dx d/dx
+        pb = kick * ( fbar * fu );
     }
-
-    // reverse: slices 0 .. n-1
-    for ( int64_t mlo = 0; mlo < int64_t( p.n ); mlo += p.chunk )
+    struct cell { int i; double t, q0, q1, q2; };
+    __device__ __forceinline__ cell locate( const double *Q ) const
     {
-        const int64_t mhi = ( mlo + p.chunk - 1 < int64_t( p.n ) - 1 ) ? mlo + p.chunk - 1 : int64_t( p.n ) - 1;
-        const int cnt = int( mhi - mlo + 1 );
-        __syncthreads();
-        dma_copy16<BLOCK>( Ql, p.qhist + size_t( mlo ) * sq, uint32_t( cnt ) * sq / 2u );
-        for ( uint32_t q = threadIdx.x; q < uint32_t( cnt ) * p.Nx; q += BLOCK ) lam[q] = 0.0;
-        dma_publish();
-        for ( int jj = 0; jj < cnt; ++jj )
-        {
-            const double hk = ( mlo + jj == 0 ) ? 0.5 * kick : kick;
-            // the cell and t the forward step used at this position
-            const double k = floor( s );
-            const double t = s - k;
-            const int i = POW2 ? ( int( k ) & mask ) : int( k );
-            double dpdt;
-            const double pv = poly_eval( Ql + jj * sq, q2, i, t, dpdt );
-            const double pbar = hk * ubar;
-            sbar = fma( pbar, dpdt, sbar );
-            if ( active )
-            {
-                // adjoints of q0 = D0 + D1, q1 = 2 (D1 - D0), q2 = D0 - 2 D1 + D2
-                const double q0 = pbar, q1 = pbar * t, q2 = pbar * ( t*t );
-                const double d0 = q0 - 2.0*q1 + q2, d1 = q0 + 2.0*q1 - 2.0*q2, d2 = q2;
-                double *L = lam + jj * p.Nx;
-                const int i0 = ( i + Nx ) % Nx;
-                atomicAdd( L + i0, -d0 );
-                atomicAdd( L + ( i0 + 1 ) % Nx, d0 - d1 );
-                atomicAdd( L + ( i0 + 2 ) % Nx, d1 - d2 );
-                atomicAdd( L + ( i0 + 3 ) % Nx, d2 );
-            }
-            // undo the step
-            u = fma( -hk, pv, u );
-            ubar = fma( -cd, sbar, ubar );
-            s = fma( cd, u, s );
-            if ( !POW2 || poly_wrap_due( mlo + jj ) ) rewrap( s, Nxd, invNx );
-        }
-        __syncthreads();
-        for ( uint32_t q = threadIdx.x; q < uint32_t( cnt ) * p.Nx; q += BLOCK )
-        {
-            const double v = lam[q];
-            if ( v != 0.0 ) atomicAdd( p.lambda + size_t( mlo ) * p.Nx + q, v );
-        }
+        cell c;
+        const double k = floor( s );
+        c.t = s - k;
+        c.i = POW2 ? ( int( k ) & mask ) : int( k );
+        const double2 q01 = reinterpret_cast<const double2*>( Q )[ c.i + 1 ];
+        c.q0 = q01.x; c.q1 = q01.y; c.q2 = Q[ q2 + ( c.i + 1 ) ];
+        return c;
     }
-}
+    __device__ __forceinline__ double undo( const cell &c, float h )
+    {
+        const double q = fma( c.q2, c.t, c.q1 ), dpdt = fma( c.q2, c.t, q ), pv = fma( q, c.t, c.q0 );
+        const double pbar = h == 1.0f ? pb : double( h ) * pb;
+        sbar = fma( pbar, dpdt, sbar );
+        u = fma( h == 1.0f ? -kick : -double( h ) * kick, pv, u );
+        pb = fma( -kick * cd, sbar, pb );
+        s = fma( cd, u, s );
+        if ( !POW2 ) wrap();
+        return pbar;
+    }
+    __device__ __forceinline__ void wrap() { rewrap( s, Nxd, invNx ); }
+};
 
-// adjoints of q0 = D0 + D1, q1 = 2 (D1 - D0), q2 = D0 - 2 D1 + D2 folded into
-// the slice adjoints of cell i (periodic, Nx points)
-__device__ __forceinline__ void scatter_poly_adjoint( double *L, int i, int Nx, double pbar, double t )
+template <bool POW2>
+struct adjoint_fp32c
 {
-    const double q0 = pbar, q1 = pbar * t, q2 = pbar * ( t*t );
-    const double d0 = q0 - 2.0*q1 + q2, d1 = q0 + 2.0*q1 - 2.0*q2, d2 = q2;
-    const int i0 = ( i + Nx ) % Nx;
-    atomicAdd( L + i0, -d0 );
-    atomicAdd( L + ( i0 + 1 ) % Nx, d0 - d1 );
-    atomicAdd( L + ( i0 + 2 ) % Nx, d1 - d2 );
-    atomicAdd( L + ( i0 + 3 ) % Nx, d2 );
-}
-
-template <int BLOCK, bool POW2>
-__global__ __launch_bounds__( BLOCK )
-void adjoint1d_fp32c_kernel( adjoint1_params p )
-{
-    extern __shared__ double lds[];
-    float  *Ql  = reinterpret_cast<float*>( lds );                       // chunk of FP32 tables
-    double *lam = lds + ( size_t( p.chunk ) * p.stride_q + 1 ) / 2;      // chunk of folded slice adjoints
-    constexpr int WPB = BLOCK / WAVE;
-    const uint32_t lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-    const uint32_t g = blockIdx.x * WPB + wave;
-    const bool task = g < p.n_tasks;
-    const uint32_t ix = task ? g / p.wpx : 0, j = task ? g % p.wpx : 0;
-    const uint32_t iu = j * WAVE + lane;
-    const bool active = task && iu < p.Nu;
-
-    const int Nx = int( p.Nx ), mask = Nx - 1;
-    const double cd = p.dt * p.dx_inv, kick = -0.5 * p.dt * p.dx_inv;
-    const uint32_t sq = p.stride_q, q2 = p.q2_off;
-    const frame1 fr = make_frame1( p.f32_p0, p.f32_w0, p.Nx );
-
-    // the FP32C trace kernel's start state (trace1d_fp32c_body)
+    using table = float;
+    double cd, kick, sbar, ubar;               // ubar: of the velocity in cells per step
+    frame1 fr;
     float sh, sl, uh, ul;
-    fp32c_start( fr, ix, cd * ( p.u_min + iu*p.du + p.du/2 ), sh, sl, uh, ul );
+    int mask;
+    uint32_t q2;
 
-    // forward: slices n-1 .. 0
-    for ( int64_t mhi = int64_t( p.n ) - 1; mhi >= 0; mhi -= p.chunk )
+    __device__ __forceinline__ static const float *tables( const adjoint1_params &p ) { return p.qhist32; }
+    __device__ __forceinline__ void start( const adjoint1_params &p, uint32_t ix, uint32_t iu )
     {
-        const int64_t mlo = mhi - int64_t( p.chunk ) + 1 > 0 ? mhi - int64_t( p.chunk ) + 1 : 0;
-        const int cnt = int( mhi - mlo + 1 );
-        __syncthreads();
-        dma_copy16<BLOCK>( Ql, p.qhist32 + size_t( mlo ) * sq, uint32_t( cnt ) * sq / 4u );
-        dma_publish();
-        for ( int jj = cnt - 1; jj >= 0; --jj )
+        cd = p.dt * p.dx_inv; kick = -0.5 * p.dt * p.dx_inv;
+        mask = int( p.Nx ) - 1; q2 = p.q2_off;
+        fr = make_frame1( p.f32_p0, p.f32_w0, p.Nx );
+        fp32c_start( fr, ix, cd * ( p.u_min + iu*p.du + p.du/2 ), sh, sl, uh, ul );
+    }
+    __device__ __forceinline__ void down( const float *Q, uint32_t sq, int mlo, int hi )
+    {
+        for ( int jj = hi; jj >= 0; --jj )
         {
-            const int64_t m = mlo + jj;
+            const int m = mlo + jj;
             if ( POW2 && poly_wrap_due( m ) ) fp32c_rewrap( fr, sh, sl, uh, ul );
             fp32c_move( fr, sh, sl, uh, ul );
             if ( !POW2 ) fp32c_rewrap( fr, sh, sl, uh, ul );
             float t;
             const int i = fp32c_locate<POW2>( fr, sh, sl, mask, t );
-            fp32c_kick( uh, ul, ( m == 0 ? 0.5f : 1.0f ) * fp32c_poly( Ql + jj * sq, q2, i, t ) );
+            fp32c_kick( uh, ul, ( m == 0 ? 0.5f : 1.0f ) * fp32c_poly( Q + jj * sq, q2, i, t ) );
         }
     }
+    __device__ __forceinline__ double foot_x( const adjoint1_params &p ) const { return p.x_min + fp32c_position( fr, sh, sl ) * p.dx; }
+    __device__ __forceinline__ double foot_u() const { return fp32c_velocity( fr, uh, ul ) / cd; }
+    __device__ __forceinline__ void seed( const adjoint1_params &p, double fbar, double fx, double fu )
+    {
+        sbar = fbar * fx * p.dx;
+        ubar = fbar * fu / cd;                 // d/dw = d/du / cd
+    }
+    struct cell { int i; float t, q0, q1, q2; };
+    __device__ __forceinline__ cell locate( const float *Q ) const
+    {
+        cell c;
+        c.i = fp32c_locate<POW2>( fr, sh, sl, mask, c.t );
+        const float2 q01 = reinterpret_cast<const float2*>( Q )[ c.i + 1 ];
+        c.q0 = q01.x; c.q1 = q01.y; c.q2 = Q[ q2 + ( c.i + 1 ) ];
+        return c;
+    }
+    __device__ __forceinline__ double undo( const cell &c, float hf )
+    {
+        const float q = fmaf( fmaf( c.q2, c.t, c.q1 ), c.t, c.q0 );
+        const double dqdt = fma( 2.0 * double( c.q2 ), double( c.t ), double( c.q1 ) );     // of the scaled table, in FP64
+        const double pbar = double( hf ) * kick * cd * ubar;
+        sbar = fma( double( hf ) * ubar, dqdt, sbar );
+        fp32c_kick( uh, ul, -( hf * q ) );     // undo the kick, then the drift
+        ubar = ubar - sbar;
+        fp32c_move<true>( fr, sh, sl, uh, ul );
+        if ( !POW2 ) wrap();
+        return pbar;
+    }
+    __device__ __forceinline__ void wrap() { fp32c_rewrap( fr, sh, sl, uh, ul ); }
+};
+
+// Sums over the wave of eight values a lane, compensated: three exchanges halve
+// the values a lane holds, three more finish its one.  Lane l gets the sum of
+// value (l >> 3) with its bits in the order 5, 4, 3, eight lanes each.
+__device__ __forceinline__ double wave_csum8( const double f[8] )
+{
+    const uint32_t lane = threadIdx.x % WAVE;
+    csum v[8];
+    #pragma unroll
+    for ( int k = 0; k < 8; ++k ) v[k] = csum { f[k], 0.0 };
+    #pragma unroll
+    for ( int half = 4, off = 32; half > 0; half >>= 1, off >>= 1 )
+    {
+        const bool up = ( lane & uint32_t( off ) ) != 0;
+        #pragma unroll
+        for ( int k = 0; k < half; ++k )
+        {
+            const csum keep = up ? v[k + half] : v[k], send = up ? v[k] : v[k + half];
+            v[k] = csum_add( keep, csum { __shfl_xor( send.s, off ), __shfl_xor( send.c, off ) } );
+        }
+    }
+    #pragma unroll
+    for ( int off = 4; off > 0; off >>= 1 )
+        v[0] = csum_add( v[0], csum { __shfl_xor( v[0].s, off ), __shfl_xor( v[0].c, off ) } );
+    return v[0].s + v[0].c;
+}
+
+// x-major nodes (lanes over consecutive x), a whole workgroup through the same
+// slices.  A node's pbar scatters into the four slice adjoints of its cell by
+// LDS atomics, issued behind the next step's table read, which they would hold
+// up.  With PIPE a slice's adjoints are a row of cells -1 .. Nx, entries 0 ..
+// Nx+4 (one address, immediate offsets), and the tables have two buffers; tables
+// too wide for two slices of that take one buffer and adjoints folded mod Nx.
+//
+// Bound by the serial chain of the steps (table read, polynomial, velocity,
+// position; about 40 of 70 us at 256 threads), then by the global atomics (15),
+// the flush's LDS passes and the LDS atomics (9 each).  128 x 512, n averaging
+// 160: with velocity-major lanes, whose 64 neighbouring velocities hit the same
+// cells, one table buffer with its copies waited for, 15-slice chunks and a
+// runtime modulo per scattered point 103 us a launch (LDS atomics 45); this one
+// 65.  The flush a row a step instead of between chunks 82 (its reads wait
+// for the scatter's queue); a cell's (pbar, pbar t, pbar t^2) scattered by three
+// atomics and combined at the flush 81.
+template <typename NODE, bool POW2, bool PIPE>
+__global__ __launch_bounds__( 1024 )
+void adjoint1d_kernel( adjoint1_params p )
+{
+    extern __shared__ __align__( 16 ) double lds[];
+    using T = typename NODE::table;
+    const uint32_t threads = blockDim.x, waves = threads / WAVE, tid = threadIdx.x;
+    const uint32_t sq = p.stride_q, C = p.chunk, Nx = p.Nx;
+    T *const Q0 = reinterpret_cast<T*>( lds ), *const Q1 = Q0 + ( PIPE ? size_t( C ) * sq : 0 );
+    double *const lam = reinterpret_cast<double*>( Q1 + size_t( C ) * sq );
+    const uint32_t lw = PIPE ? Nx + 5 : Nx;                        // adjoints per slice
+    const T *const hist = NODE::tables( p );
+
+    const uint64_t nodes = uint64_t( Nx ) * p.Nu, q = uint64_t( blockIdx.x ) * threads + tid;
+    const bool active = q < nodes;
+    const uint64_t qn = q < nodes ? q : q % nodes;                 // lanes past the last node repeat others with weight 0
+    const uint32_t iu = uint32_t( qn / Nx ), ix = uint32_t( qn - uint64_t( iu ) * Nx );
+    // this wave's gradient sums, one value a lane (wave_csum8)
+    const uint32_t wave = blockIdx.x * waves + tid / WAVE, l8 = tid % WAVE / 8;
+    const uint32_t par = ( l8 >> 2 ) * 4 + ( ( l8 >> 1 ) & 1 ) * 2 + ( l8 & 1 );
+    double *const grad = p.grad_part + size_t( wave ) * NUFI_MAX_MODES + par;
+    const bool keeps = tid % 8 == 0 && wave < p.n_tasks && par < p.npar;
+    const double grad0 = keeps ? *grad : 0.0, gx = p.g[ix];
+    NODE nd;
+    nd.start( p, ix, iu );
+
+    // forward: slices n-1 .. 0, the steps of the trace kernel
+    auto down = [&]( const T *Q, int mlo, int hi, int ) __attribute__(( always_inline )) { nd.down( Q, sq, mlo, hi ); };
+    if ( PIPE ) poly_ready_pipeline( Q0, hist, sq, p.n, C, waves, down );
+    else        poly_ready_direct( Q0, hist, sq, p.n, C, waves, down );
+
+    // the reverse sweep's first tables come while the seeds are formed
+    const int n = int( p.n ), Ci = int( C ), K = ( n + Ci - 1 ) / Ci;
+    auto cnt_of = [&]( int k ) { return n - k * Ci < Ci ? n - k * Ci : Ci; };
+    auto copy = [&]( T *dst, int k ) __attribute__(( always_inline ))
+    {
+        dma_copy16( dst, hist + size_t( k ) * C * sq, uint32_t( cnt_of( k ) ) * ( sq * uint32_t( sizeof( T ) ) / 16u ), waves );
+    };
+    __syncthreads();                                        // the forward chunks are read
+    if ( K > 0 ) copy( Q0, 0 );
+    for ( uint32_t e = tid; e < C * lw; e += threads ) lam[e] = 0.0;
 
     // seed at the foot
-    const double fbar = active ? -p.du * p.g[ix] : 0.0;
-    double fx, fu, fa[NUFI_MAX_MODES];
-    f0_grad_1d( p.f0, p.x_min + fp32c_position( fr, sh, sl ) * p.dx, fp32c_velocity( fr, uh, ul ) / cd,
-                fx, fu, fa, p.npar );
-    double sbar = fbar * fx * p.dx;     // d/ds = dx d/dx
-    double ubar = fbar * fu / cd;       // d/dw = d/du / cd
-    #pragma unroll
-    for ( int m = 0; m < NUFI_MAX_MODES; ++m )
     {
-        if ( m >= int( p.npar ) ) continue;
-        const csum v = wave_csum( csum { fbar * fa[m], 0.0 } );
-        if ( task && lane == 0 ) p.grad_part[ size_t( g ) * NUFI_MAX_MODES + m ] += v.s + v.c;
+        static_assert( NUFI_MAX_MODES == 8, "wave_csum8" );
+        const double fbar = active ? -p.du * gx : 0.0;
+        double fx, fu, fa[NUFI_MAX_MODES] = { 0, 0, 0, 0, 0, 0, 0, 0 };
+        f0_grad_1d( p.f0, nd.foot_x( p ), nd.foot_u(), fx, fu, fa, p.npar );
+        nd.seed( p, fbar, fx, fu );
+        #pragma unroll
+        for ( int m = 0; m < NUFI_MAX_MODES; ++m ) fa[m] *= fbar;
+        const double sum = wave_csum8( fa );
+        if ( keeps ) *grad = grad0 + sum;
     }
 
-    // reverse: slices 0 .. n-1, undoing each step on the pairs
-    for ( int64_t mlo = 0; mlo < int64_t( p.n ); mlo += p.chunk )
+    // reverse: slices 0 .. n-1 in chunks
+    auto scatter = [&]( double *L, int i, double t, double pbar ) __attribute__(( always_inline ))
     {
-        const int64_t mhi = ( mlo + p.chunk - 1 < int64_t( p.n ) - 1 ) ? mlo + p.chunk - 1 : int64_t( p.n ) - 1;
-        const int cnt = int( mhi - mlo + 1 );
-        __syncthreads();
-        dma_copy16<BLOCK>( Ql, p.qhist32 + size_t( mlo ) * sq, uint32_t( cnt ) * sq / 4u );
-        for ( uint32_t q = threadIdx.x; q < uint32_t( cnt ) * p.Nx; q += BLOCK ) lam[q] = 0.0;
-        dma_publish();
-        for ( int jj = 0; jj < cnt; ++jj )
+        // adjoints of q0 = D0 + D1, q1 = 2 (D1 - D0), q2 = D0 - 2 D1 + D2, Dl = c[i+l] - c[i+l-1] of the row from c[i]
+        const double q0 = pbar, q1 = pbar * t, q2 = q1 * t;
+        const double n0 = fma( 2.0, q1, -fma( q1, t, q0 ) ), d1 = fma( 2.0, q1 - q2, q0 );         // n0 = -d0
+        uint32_t e = uint32_t( i + 1 );
+        if ( PIPE )
         {
-            const int64_t m = mlo + jj;
-            const float hf = m == 0 ? 0.5f : 1.0f;
-            const float *Q = Ql + jj * sq;
-            float t;
-            const int i = fp32c_locate<POW2>( fr, sh, sl, mask, t );
-            const float q = fp32c_poly( Q, q2, i, t );
-            // dq/dt of the scaled table, in FP64
-            const float2 q01 = reinterpret_cast<const float2*>( Q )[ i + 1 ];
-            const double dqdt = fma( 2.0 * double( Q[ q2 + ( i + 1 ) ] ), double( t ), double( q01.y ) );
-            const double pbar = double( hf ) * kick * cd * ubar;
-            sbar = fma( double( hf ) * ubar, dqdt, sbar );
-            if ( active ) scatter_poly_adjoint( lam + jj * p.Nx, i, Nx, pbar, double( t ) );
-            // undo the kick, then the drift
-            fp32c_kick( uh, ul, -( hf * q ) );
-            ubar = ubar - sbar;
-            fp32c_move<true>( fr, sh, sl, uh, ul );
-            if ( !POW2 || poly_wrap_due( m ) ) fp32c_rewrap( fr, sh, sl, uh, ul );
+            atomicAdd( L + e, n0 );          atomicAdd( L + e + 1, -n0 - d1 );
+            atomicAdd( L + e + 2, d1 - q2 ); atomicAdd( L + e + 3, q2 );
+            return;
         }
-        __syncthreads();
-        for ( uint32_t q = threadIdx.x; q < uint32_t( cnt ) * p.Nx; q += BLOCK )
+        e = i < 0 ? Nx - 1 : uint32_t( i );                 // a ring may be shorter than the four points
+        if ( e >= Nx ) e -= Nx;
+        auto next = [&]() { if ( ++e == Nx ) e = 0; };
+        atomicAdd( L + e, n0 );       next();
+        atomicAdd( L + e, -n0 - d1 ); next();
+        atomicAdd( L + e, d1 - q2 );  next();
+        atomicAdd( L + e, q2 );
+    };
+    // the chunk's adjoints to global memory, and cleared: a wave takes whole rows.
+    // PIPE: entries 0 and Nx+1 .. Nx+4 lie a period off and go by themselves.
+    auto flush = [&]( uint32_t cnt, double *to ) __attribute__(( always_inline ))
+    {
+        const uint32_t w = __builtin_amdgcn_readfirstlane( tid / WAVE );
+        for ( uint32_t jj = w; jj < cnt; jj += waves )
         {
-            const double v = lam[q];
-            if ( v != 0.0 ) atomicAdd( p.lambda + size_t( mlo ) * p.Nx + q, v );
+            double *S = lam + jj * lw + ( PIPE ? 1 : 0 ), *G = to + jj * Nx;
+            for ( uint32_t x = tid % WAVE; x < Nx; x += WAVE )
+            {
+                const double v = S[x];
+                S[x] = 0.0;
+                atomicAdd( G + x, v );
+            }
         }
+        if ( !PIPE ) return;
+        for ( uint32_t e = tid; e < cnt * 5; e += threads )
+        {
+            const uint32_t jj = e / 5, c = e - jj * 5;
+            double *S = lam + jj * lw + ( c == 4 ? 0u : Nx + 1 + c );
+            const double v = *S;
+            *S = 0.0;
+            if ( v != 0.0 ) atomicAdd( to + jj * Nx + ( c == 4 ? Nx - 1 : c % Nx ), v );
+        }
+    };
+    dma_publish();
+    for ( int k = 0; k < K; ++k )
+    {
+        const int cnt = cnt_of( k ), mlo = k * Ci;
+        const T *Q = ( PIPE && ( k & 1 ) ) ? Q1 : Q0;
+        if ( PIPE && k + 1 < K ) copy( ( k & 1 ) ? Q0 : Q1, k + 1 );
+        // the pending adjoints: of the step before, at first zeros
+        double *L = lam, *now = lam, tp = 0.0, pp = 0.0;
+        int ip = int( ix ), jj = 0;
+        auto step = [&]( float h ) __attribute__(( always_inline ))
+        {
+            const auto c = nd.locate( Q );
+            __builtin_amdgcn_sched_barrier( 0 );
+            scatter( L, ip, tp, pp );
+            __builtin_amdgcn_sched_barrier( 0 );
+            pp = nd.undo( c, h );
+            tp = double( c.t ); ip = c.i;
+            L = now; now += lw;
+            Q += sq; ++jj;
+        };
+        if ( mlo == 0 ) step( 0.5f );
+        while ( jj < cnt )                                  // segments between re-wrap points
+        {
+            const int left = POLY_WRAP - ( ( mlo + jj ) & ( POLY_WRAP - 1 ) );
+            const int stop = POW2 && jj + left < cnt ? jj + left : cnt;
+            while ( jj < stop ) step( 1.0f );
+            if ( POW2 && poly_wrap_due( mlo + jj - 1 ) ) nd.wrap();
+        }
+        scatter( L, ip, tp, pp );
+        if ( PIPE ) dma_publish();                          // the adjoints are complete and the next tables there
+        else
+        {
+            __syncthreads();
+            if ( k + 1 < K ) copy( Q0, k + 1 );
+        }
+        flush( uint32_t( cnt ), p.lambda + size_t( mlo ) * Nx );
+        if ( PIPE ) __syncthreads();
+        else        dma_publish();
     }
 }
 
@@ -353,34 +457,52 @@ void reduce_grad_kernel( const double *part, uint32_t n_tasks, uint32_t npar, do
 
 } // namespace
 
-size_t adjoint1d_lds_bytes( const adjoint1_params &p )
+// Workgroups of 512 threads, 1024 where a CU would get two of them: one takes
+// the whole LDS.  Fewer workgroups add fewer global atomics (each adds to every
+// slice adjoint) and longer LDS queues: at 128 x 512, 256 threads (every CU)
+// 70 us, 512 (half of them) 65, 1024 103.  Two table buffers and padded adjoint rows where at least two slices of both fit.
+void plan_adjoint1d( adjoint1_params &p, int n_cu, size_t lds_cap )
 {
-    if ( p.qhist32 ) return ( size_t( p.chunk ) * p.stride_q + 1 ) / 2 * sizeof(double) + size_t( p.chunk ) * p.Nx * sizeof(double);
-    return size_t( p.chunk ) * ( p.stride_q + p.Nx ) * sizeof(double);
+    const uint64_t nodes = uint64_t( p.Nx ) * p.Nu;
+    p.threads = 512;
+    while ( p.threads < 1024 && nodes > uint64_t( p.threads ) * uint64_t( n_cu ) ) p.threads *= 2;
+    const size_t table = size_t( p.stride_q ) * ( p.qhist32 ? sizeof(float) : sizeof(double) );
+    const size_t cap = std::min<size_t>( lds_cap, 160 * 1024 ), two = 2 * table + 8 * ( size_t( p.Nx ) + 5 );
+    p.pipe = cap / two >= 2;
+    const size_t per = p.pipe ? two : table + size_t( p.Nx ) * sizeof(double);
+    p.chunk = uint32_t( std::max<size_t>( 1, std::min<size_t>( 32, cap / per ) ) );
 }
 
-hipError_t launch_adjoint1d( const adjoint1_params &p, hipStream_t st )
+size_t adjoint1d_lds_bytes( const adjoint1_params &p )
 {
-    if ( p.n_tasks == 0 ) return hipSuccess;
-    constexpr int BLOCK = 256;
-    const uint32_t grid = ( p.n_tasks + BLOCK / WAVE - 1 ) / ( BLOCK / WAVE );
+    const size_t table = size_t( p.stride_q ) * ( p.qhist32 ? sizeof(float) : sizeof(double) );
+    return size_t( p.chunk ) * ( p.pipe ? 2 * table + 8 * ( size_t( p.Nx ) + 5 ) : table + size_t( p.Nx ) * sizeof(double) );
+}
+
+template <bool POW2, bool PIPE>
+static const void *adjoint1d_entry( bool f32 )
+{
+    return f32 ? reinterpret_cast<const void*>( adjoint1d_kernel<adjoint_fp32c<POW2>,POW2,PIPE> )
+               : reinterpret_cast<const void*>( adjoint1d_kernel<adjoint_fp64<POW2>,POW2,PIPE> );
+}
+
+hipError_t launch_adjoint1d( const adjoint1_params &p_in, hipStream_t st )
+{
+    adjoint1_params p = p_in;
+    const uint64_t nodes = uint64_t( p.Nx ) * p.Nu, grid = ( nodes + p.threads - 1 ) / p.threads;
+    if ( nodes == 0 ) return hipSuccess;
     const size_t lds = adjoint1d_lds_bytes( p );
-    const bool pow2 = ( p.Nx & ( p.Nx - 1 ) ) == 0;
-    const bool f32 = p.qhist32 != nullptr;
-    const void *k = f32 ? ( pow2 ? reinterpret_cast<const void*>( adjoint1d_fp32c_kernel<BLOCK,true> )
-                                 : reinterpret_cast<const void*>( adjoint1d_fp32c_kernel<BLOCK,false> ) )
-                        : ( pow2 ? reinterpret_cast<const void*>( adjoint1d_kernel<BLOCK,true> )
-                                 : reinterpret_cast<const void*>( adjoint1d_kernel<BLOCK,false> ) );
+    const bool pow2 = ( p.Nx & ( p.Nx - 1 ) ) == 0, f32 = p.qhist32 != nullptr;
+    const void *k = p.pipe ? ( pow2 ? adjoint1d_entry<true,true>( f32 ) : adjoint1d_entry<false,true>( f32 ) )
+                            : ( pow2 ? adjoint1d_entry<true,false>( f32 ) : adjoint1d_entry<false,false>( f32 ) );
     if ( lds > 65536 )
     {
         hipError_t e = hipFuncSetAttribute( k, hipFuncAttributeMaxDynamicSharedMemorySize, int( lds ) );
         if ( e != hipSuccess ) return e;
     }
-    if ( f32 && pow2 )  hipLaunchKernelGGL( ( adjoint1d_fp32c_kernel<BLOCK,true> ), dim3( grid ), dim3( BLOCK ), lds, st, p );
-    else if ( f32 )     hipLaunchKernelGGL( ( adjoint1d_fp32c_kernel<BLOCK,false> ), dim3( grid ), dim3( BLOCK ), lds, st, p );
-    else if ( pow2 )    hipLaunchKernelGGL( ( adjoint1d_kernel<BLOCK,true> ), dim3( grid ), dim3( BLOCK ), lds, st, p );
-    else                hipLaunchKernelGGL( ( adjoint1d_kernel<BLOCK,false> ), dim3( grid ), dim3( BLOCK ), lds, st, p );
-    return hipGetLastError();
+    void *args[] = { &p };
+    const hipError_t e = hipLaunchKernel( k, dim3( uint32_t( grid ) ), dim3( p.threads ), args, lds, st );
+    return e != hipSuccess ? e : hipGetLastError();
 }
 
 hipError_t launch_adjoint_field( const adjoint_field_params &p, hipStream_t st )

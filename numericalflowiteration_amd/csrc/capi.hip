@@ -885,8 +885,7 @@ int nufi_adjoint_grad( nufi_ctx *c, double *dJ_da, int n_par, double *J_out )
     ap.u_min = c->conf.u_min; ap.du = c->conf.du; ap.f0 = c->conf.f0;
     fp32c_frame( double( Nx ), c->conf.dt * c->conf.dx_inv, c->conf.u_min, double( c->conf.Nu ), c->conf.du,
                  ap.f32_p0, ap.f32_w0 );
-    const size_t per_slice = size_t( c->sq ) * ( f32 ? sizeof(float) : sizeof(double) ) + Nx * sizeof(double);
-    ap.chunk = uint32_t( std::max<size_t>( 1, std::min<size_t>( 32, std::min<size_t>( c->lds_cap, 65536 ) / per_slice ) ) );
+    plan_adjoint1d( ap, c->n_cu, c->lds_cap );
     if ( adjoint1d_lds_bytes( ap ) > LDS_LIMIT )
         return fail( c, NUFI_ERR_UNSUPPORTED, "adjoint_grad: one slice's tables and adjoints exceed the LDS" );
     for ( uint64_t n = Nt + 1; n-- > 0; )

@@ -277,9 +277,10 @@ struct adjoint1_params
     const float  *qhist32;    // FP32C: the FP32 tables scaled by the kick (qhist is then null)
     const double *g;          // dJ/drho_n (Nx)
     double       *lambda;     // folded slice adjoints, slice m at lambda + m*Nx
-    double       *grad_part;  // per wave-task parameter-gradient accumulators [g][NUFI_MAX_MODES]
+    double       *grad_part;  // per wave parameter-gradient accumulators [g][NUFI_MAX_MODES], n_tasks of them
     uint64_t n;
     uint32_t Nx, Nu, stride_d, stride_q, q2_off, wpx, n_tasks, chunk, npar;
+    uint32_t threads, pipe;   // plan_adjoint1d: workgroup size; two table buffers and padded adjoint rows
     double x_min, dx, dx_inv, dt, u_min, du;
     float f32_p0, f32_w0;     // FP32C: the trace kernel's frames (fp32c_frame)
     nufi_f0 f0;
@@ -295,6 +296,8 @@ struct adjoint_field_params
     double dt;
 };
 
+// threads, pipe and chunk from the grid, the tables' type and the LDS
+void plan_adjoint1d( adjoint1_params &p, int n_cu, size_t lds_cap );
 hipError_t launch_adjoint1d( const adjoint1_params &p, hipStream_t st );
 size_t adjoint1d_lds_bytes( const adjoint1_params &p );
 hipError_t launch_adjoint_field( const adjoint_field_params &p, hipStream_t st );

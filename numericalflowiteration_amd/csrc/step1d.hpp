@@ -82,14 +82,6 @@ __device__ __forceinline__ int poly_locate( double &x, int mask, double Nxd, dou
     return wrap_locate( x, Nxd, invNx, t );
 }
 
-__device__ __forceinline__ double poly_eval( const double *Q, uint32_t q2, int i, double t, double &dpdt )
-{
-    const double2 q01 = reinterpret_cast<const double2*>( Q )[ i + 1 ];
-    const double c2 = Q[ q2 + ( i + 1 ) ];
-    dpdt = fma( 2.0 * c2, t, q01.y );
-    return fma( fma( c2, t, q01.y ), t, q01.x );
-}
-
 // Q: the slice's pairs, Q2: its Q2 row (Q + q2)
 template <bool POW2>
 __device__ __forceinline__ void poly_step( double &s, double &u, const double *Q, const double *Q2, double cd,
