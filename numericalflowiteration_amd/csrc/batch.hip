@@ -284,6 +284,8 @@ int nufi_batch_create( const nufi_config *confs, uint64_t n_runs, int order, int
         f.Nx = uint32_t( c.Nx ); f.Ny = 1; f.Nz = 1; f.N = uint32_t( c.Nx );
         uint32_t l2 = 0; while ( ( uint64_t( 1 ) << l2 ) < c.Nx ) ++l2;
         f.log2x = ( ( c.Nx & ( c.Nx - 1 ) ) == 0 ) ? l2 : 0xffffffffu;
+        f.rx = make_radices( uint32_t( c.Nx ), precision == NUFI_FP32C );
+        f.sum_group = field_sum_group( c.Nx, precision == NUFI_FP32C );
         f.log2y = 0; f.log2z = 0;
         f.partials = p.partials; f.wpx = b->wpx[r]; f.weight = -c.du; f.tw_lds = tw_lds;
         f.tw_x = b->tw + b->off_tab[r]; f.tw_y = f.tw_x; f.tw_z = f.tw_x;

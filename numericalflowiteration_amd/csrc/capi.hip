@@ -368,6 +368,9 @@ field_params base_field( nufi_ctx *c )
     f.Nz = c->dim == 3 ? uint32_t( c->conf.Nz ) : 1u;
     f.N = f.Nx * f.Ny * f.Nz;
     f.log2x = log2_or_none( f.Nx ); f.log2y = log2_or_none( f.Ny ); f.log2z = log2_or_none( f.Nz );
+    const bool fp32c = c->precision == NUFI_FP32C;
+    f.rx = make_radices( f.Nx, fp32c ); f.ry = make_radices( f.Ny, fp32c ); f.rz = make_radices( f.Nz, fp32c );
+    f.sum_group = field_sum_group( f.N, fp32c );
     f.wpx = rho_ppx( c );
     f.weight = rho_weight( c );
     f.tw_x = c->tw_x; f.tw_y = c->tw_y; f.tw_z = c->tw_z;
@@ -597,7 +600,7 @@ int nufi_compute_rho( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_end 
     if ( q_begin == q_end )
     {
         // empty range: the device rho becomes zero, so download_rho adds nothing
-        hipError_t e = launch_reduce_partials( c->partials, rho_ppx( c ), 0.0, 0, 0, uint32_t( c->n_space ), c->rho, c->stream );
+        hipError_t e = launch_reduce_partials( c->partials, rho_ppx( c ), 0.0, 0, 0, uint32_t( c->n_space ), 1, c->rho, c->stream );
         if ( e != hipSuccess ) return hip_fail( c, e, "reduce launch" );
         return NUFI_OK;
     }
@@ -605,7 +608,8 @@ int nufi_compute_rho( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_end 
     int rc = launch_trace( c, n, q_begin, q_end, &first, &count );
     if ( rc ) return rc;
     hipError_t e = launch_reduce_partials( c->partials, rho_ppx( c ), rho_weight( c ), uint32_t( first ), uint32_t( count ),
-                                           uint32_t( c->n_space ), c->rho, c->stream );
+                                           uint32_t( c->n_space ), field_sum_group( c->n_space, c->precision == NUFI_FP32C ),
+                                           c->rho, c->stream );
     if ( e != hipSuccess ) return hip_fail( c, e, "reduce launch" );
     return NUFI_OK;
 }
@@ -739,7 +743,7 @@ static int step_async( nufi_ctx *c, uint64_t n, double *rho_out )
         // in the same order, and the single field workgroup starts from rho
         double *dst = rho_out ? rho_out : c->rho;
         hipError_t e = launch_reduce_partials( c->partials, f.wpx, f.weight, 0, uint32_t( c->n_space ),
-                                               uint32_t( c->n_space ), dst, c->stream );
+                                               uint32_t( c->n_space ), f.sum_group, dst, c->stream );
         if ( e != hipSuccess ) return hip_fail( c, e, "reduce launch" );
         f.partials = nullptr;
         f.values = dst;
@@ -871,7 +875,7 @@ int nufi_adjoint_grad( nufi_ctx *c, double *dJ_da, int n_par, double *J_out )
     HIP_TRY( c, hipMemsetAsync( c->grad_part, 0, size_t( n_tasks ) * NUFI_MAX_MODES * sizeof(double), c->stream ) );
 
     adjoint_field_params af {};
-    af.N = uint32_t( Nx ); af.log2x = log2_or_none( Nx );
+    af.N = uint32_t( Nx ); af.log2x = log2_or_none( Nx ); af.rx = make_radices( af.N );
     af.g = c->gvec; af.tw = c->tw_x; af.mult = c->mult_step; af.ewt = c->ewt; af.dt = c->conf.dt;
     adjoint1_params ap {};
     const bool f32 = c->precision == NUFI_FP32C;

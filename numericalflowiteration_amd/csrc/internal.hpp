@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "../../include/nufi_hip.h"
+#include "fft_lds.hpp"
 
 namespace nufi_impl
 {
@@ -289,11 +290,13 @@ struct adjoint1_params
 struct adjoint_field_params
 {
     uint32_t N, log2x;
+    fft_radices rx;
     const double  *rho, *lambda;   // rho_n and lambda_n (Nx)
     double        *g;              // out: dJ/drho_n
     const double2 *tw, *mult;      // twiddles, step multiplier
     const double  *ewt;
     double dt;
+    uint32_t wide;                 // one transform at a time (set by the launcher)
 };
 
 // threads, pipe and chunk from the grid, the tables' type and the LDS
@@ -340,6 +343,8 @@ struct field_params
     int      dim, order, mode;
     uint32_t Nx, Ny, Nz, N;      // N = Nx*Ny*Nz
     uint32_t log2x, log2y, log2z; // 0xffffffff if not a power of two
+    fft_radices rx, ry, rz;      // their stages then
+    uint32_t sum_group;          // threads that share a point's partial sums (field_sum_group)
     const double *partials;      // FIELD_STEP: partials (nullable -> use values)
     uint32_t wpx;
     double   weight;             // -dv multiplier applied to partial sums
@@ -360,6 +365,13 @@ struct field_params
     uint32_t sy, sz, stride_d;
 };
 
+// Threads that share the partial sums of a point: with few points the idle
+// ones of a FIELD_BLOCK workgroup, at most 8; one in FP32C.
+inline uint32_t field_sum_group( size_t n, bool fp32c )
+{
+    if ( fp32c ) return 1;
+    return n * 8 <= FIELD_BLOCK ? 8u : n * 4 <= FIELD_BLOCK ? 4u : n * 2 <= FIELD_BLOCK ? 2u : 1u;
+}
 hipError_t launch_field( const field_params &p, hipStream_t st );
 // The same solve over many workgroups for grids field_supported refuses
 // (field_large.hip): W0, W1 hold N complex values each, epart
@@ -389,8 +401,8 @@ hipError_t launch_reduce_metrics( const double *partials, uint32_t n_tasks, doub
 // Sum of the partials into rho[ix] = weight * sum_j partials[j*n_space + ix]
 // for ix in [first, first+count), zero elsewhere (n_space entries).
 hipError_t launch_reduce_partials( const double *partials, uint32_t wpx, double weight,
-                                   uint32_t first, uint32_t count, uint32_t n_space,
-                                   double *rho, hipStream_t st );
+                                   uint32_t first, uint32_t count, uint32_t n_space, uint32_t G,
+                                   double *rho, hipStream_t st );       // G: field_sum_group
 // The 1D FP32C trace carries its velocities in cells per step (w = dt dx_inv
 // u): its FP32 kick-polynomial tables are scaled in FP64 by the kick
 // -dt dx_inv / 2 times dt dx_inv before their one rounding.

@@ -120,7 +120,7 @@ extern "C" int nufi_rho3d_noalloc( const nufi_config *conf, uint64_t n, const do
     hipError_t e = launch_trace3d( p, TRACE_FAST, launch_shape { 512, zc.ok ? 8 : 4, 1 }, s );
     if ( e != hipSuccess ) return fail( NUFI_ERR_DEVICE, std::string( "rho3d_noalloc: trace launch: " ) + hipGetErrorString( e ) );
     e = launch_reduce_partials( part, uint32_t( ppx ), -( conf->du * conf->dv * conf->dw ), 0, uint32_t( n_space ),
-                                uint32_t( n_space ), rho_dev, s );
+                                uint32_t( n_space ), field_sum_group( n_space, false ), rho_dev, s );
     if ( e != hipSuccess ) return fail( NUFI_ERR_DEVICE, std::string( "rho3d_noalloc: reduce launch: " ) + hipGetErrorString( e ) );
     return NUFI_OK;
 }
