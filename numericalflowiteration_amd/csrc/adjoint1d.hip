@@ -116,16 +116,7 @@ struct adjoint_fp64
     }
     __device__ __forceinline__ void down( const double *Q, uint32_t sq, int mlo, int hi )
     {
-        for ( int jj = hi; jj >= 0; )          // segments between re-wrap points
-        {
-            if ( POW2 && poly_wrap_due( mlo + jj ) ) rewrap( s, Nxd, invNx );
-            const int jstop = POW2 ? int( poly_segment_end( mlo + jj, mlo ) ) - mlo : -1;
-            const int half = mlo == 0 && jstop < 0 ? 1 : 0;          // slice 0, the last of its segment
-            const double *R = Q + jj * sq;
-            #pragma unroll 4
-            for ( ; jj >= jstop + 1 + half; --jj, R -= sq ) poly_step<POW2>( s, u, R, R + q2, cd, kick, mask, Nxd, invNx );
-            if ( half ) { poly_step<POW2>( s, u, Q, Q + q2, cd, 0.5 * kick, mask, Nxd, invNx ); --jj; }
-        }
+        poly_down<POW2>( s, u, Q, sq, q2, mlo, hi, cd, kick, mask, Nxd, invNx );
     }
     __device__ __forceinline__ double foot_x( const adjoint1_params &p ) const { return p.x_min + s*p.dx; }
     __device__ __forceinline__ double foot_u() const { return u; }

@@ -676,7 +676,15 @@ int nufi_compute_metrics( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_
             p.weight = m.du * m.dx;                                // cuda_kernel.cu:71
             p.f0 = g.f0;
             const int chunk = int( std::max<size_t>( 1, std::min<size_t>( 64, std::min<size_t>( c->lds_cap, 65536 ) / ( size_t( c->sd ) * 8 ) ) ) );
-            e = launch_trace1d( p, variant, launch_shape { 256, 1, chunk }, c->n_cu, c->stream );
+            if ( variant == TRACE_FAST && c->order == 4 && c->qhist != nullptr && trace1d_metrics_ok( p.Nx ) )
+            {
+                uint32_t waves = 0;
+                p.qhist = c->qhist; p.stride_q = c->sq; p.q2_off = poly_q2( p.Nx ); p.kick = -0.5 * g.dt * g.dx_inv;
+                p.ix_count = uint32_t( l1 - l0 + 1 );
+                e = launch_trace1d_metrics( p, c->n_cu, c->lds_cap, &waves, c->stream );
+                tasks = waves;
+            }
+            else e = launch_trace1d( p, variant, launch_shape { 256, 1, chunk }, c->n_cu, c->stream );
         }
         else
         {

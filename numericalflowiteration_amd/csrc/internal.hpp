@@ -235,6 +235,9 @@ struct launch_shape
 
 // Launchers (trace1d.hip / trace3d.hip).  Return hipSuccess or the error.
 hipError_t launch_trace1d( const trace1_params &p, int variant, const launch_shape &s, int n_cu, hipStream_t st );
+// FP64 metrics from the kick-polynomial tables where one fits the LDS; *tasks: partials written
+bool trace1d_metrics_ok( uint32_t Nx );
+hipError_t launch_trace1d_metrics( const trace1_params &p, int n_cu, size_t lds_cap, uint32_t *tasks, hipStream_t st );
 hipError_t launch_trace3d( const trace3_params &p, int variant, const launch_shape &s, hipStream_t st );
 // The z-cell kernel for grids whose window fits the LDS (ok = false
 // otherwise): its groups depend on the grid alone.  *tasks: metrics partials written.

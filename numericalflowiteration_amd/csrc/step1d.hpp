@@ -96,6 +96,24 @@ __device__ __forceinline__ void poly_step( double &s, double &u, const double *Q
     s = x;
 }
 
+// steps of slices mlo+hi .. mlo of one node, tables of sq elements each at Q, in
+// segments between re-wrap points (slice 0, the last of its segment, half)
+template <bool POW2>
+__device__ __forceinline__ void poly_down( double &s, double &u, const double *Q, uint32_t sq, uint32_t q2, int mlo, int hi,
+                                           double cd, double kick, int mask, double Nxd, double invNx )
+{
+    for ( int jj = hi; jj >= 0; )
+    {
+        if ( POW2 && poly_wrap_due( mlo + jj ) ) s = fma( -Nxd, floor( s * invNx ), s );
+        const int jstop = POW2 ? int( poly_segment_end( mlo + jj, mlo ) ) - mlo : -1;
+        const int half = mlo == 0 && jstop < 0 ? 1 : 0;
+        const double *R = Q + jj * sq;
+        #pragma unroll 4
+        for ( ; jj >= jstop + 1 + half; --jj, R -= sq ) poly_step<POW2>( s, u, R, R + q2, cd, kick, mask, Nxd, invNx );
+        if ( half ) { poly_step<POW2>( s, u, Q, Q + q2, cd, 0.5 * kick, mask, Nxd, invNx ); --jj; }
+    }
+}
+
 // ---- the FP32-compensated step ---------------------------------------------
 // Position (cell units) and velocity (cells per step, w = dt dx_inv u) as
 // unevaluated pairs (hi + lo) whose hi parts carry the offsets P0 and W0 of

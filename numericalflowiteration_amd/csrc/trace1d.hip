@@ -377,6 +377,47 @@ void trace1d_poly_kernel( trace1_params p )
     trace1d_poly_body<NPT,POW2,BLOCK>( p, blockIdx.x, lds );
 }
 
+// ---- FP64 metrics on the tables ------------------------------------------------
+// eval_f (initial half-kick from slice n, read from global memory) on the metrics
+// grid, x-major: lanes over consecutive x of one velocity, and so on to the next
+// row; the slices below n as in the rho trace.  Bound like it by the step's
+// chain and LDS reads.  256 x 1024 nodes, n = 400: velocity-major lanes over the
+// difference slices (trace1d_fast_kernel, one buffer) 181 us, this 85.
+template <bool POW2>
+__global__ __launch_bounds__( 1024 )
+void trace1d_metrics_kernel( trace1_params p )
+{
+    extern __shared__ double lds[];
+    const uint32_t waves = blockDim.x / WAVE;
+    const uint64_t nodes = uint64_t( p.ix_count ) * p.Nu, k = uint64_t( blockIdx.x ) * blockDim.x + threadIdx.x;
+    const uint64_t kn = k < nodes ? k : 0;
+    const uint32_t iu = uint32_t( kn / p.ix_count ), ix = p.ix_first + uint32_t( kn - uint64_t( iu ) * p.ix_count );
+    const uint64_t q = uint64_t( ix ) * p.Nu + iu;
+    const bool active = k < nodes && q >= p.q_begin && q < p.q_end;
+    const double Nxd = double( p.Nx ), invNx = 1.0 / Nxd, cd = p.dt * p.dx_inv;
+    const int mask = int( p.Nx ) - 1;
+    const uint32_t sq = p.stride_q, q2 = p.q2_off;
+    const double u0 = p.nu_min + iu*p.ndu + p.ndu/2;            // cuda_kernel.cu:70
+    double s = ( ( p.nx_min + ix*p.ndx ) - p.x_min ) * p.dx_inv, u = u0;
+    if ( p.n > 0 )
+    {
+        const double *Q = p.qhist + size_t( p.n ) * sq;
+        double t;
+        const int i = wrap_locate( s, Nxd, invNx, t );
+        const double2 q01 = reinterpret_cast<const double2*>( Q )[ i + 1 ];
+        u = fma( 0.5 * p.kick, fma( fma( Q[ q2 + ( i + 1 ) ], t, q01.y ), t, q01.x ), u );
+        auto steps = [&]( const double *C, int mlo, int hi, int )
+        {
+            poly_down<POW2>( s, u, C, sq, q2, mlo, hi, cd, p.kick, mask, Nxd, invNx );
+        };
+        if ( p.pipe ) poly_ready_pipeline( lds, p.qhist, sq, p.n, p.chunk, waves, steps );
+        else          poly_ready_direct( lds, p.qhist, sq, p.n, p.chunk, waves, steps );
+    }
+    const double f = active ? f0_1d( p.f0, p.x_min + s*p.dx, u ) : 0.0;
+    const uint32_t g = blockIdx.x * waves + threadIdx.x / WAVE;
+    write_metrics( p.partials, g, g < p.n_tasks, active, p.weight, f, u0*u0 );
+}
+
 // ---- FP32 compensated (order 4) --------------------------------------------
 // The FP32 kick-polynomial table: an 8-byte (Q0, Q1) and a 4-byte Q2 LDS
 // read per char-step.
@@ -692,6 +733,30 @@ size_t trace1d_lds_bytes( const trace1_params &p, int variant, const launch_shap
     // x-major: the f values of the workgroup (at most block*npt doubles) reuse the LDS
     const size_t fbuf = x_major( p, variant ) ? size_t( s.block ) * size_t( s.npt ) * sizeof(double) : 0;
     return hist > fbuf ? hist : fbuf;
+}
+
+// Workgroups of 256 threads, 512 or 1024 where a CU would get two: each CU copies
+// every slice once.  Grids whose table does not fit the LDS are refused (the
+// caller's fast kernel takes them).
+bool trace1d_metrics_ok( uint32_t Nx ) { return size_t( poly_stride( Nx ) ) * sizeof(double) <= 160u * 1024u; }
+
+hipError_t launch_trace1d_metrics( const trace1_params &p_in, int n_cu, size_t lds_cap, uint32_t *tasks, hipStream_t st )
+{
+    trace1_params p = p_in;
+    const uint64_t nodes = uint64_t( p.ix_count ) * p.Nu;
+    if ( p.qhist == nullptr || nodes == 0 || p.n >= ( uint64_t( 1 ) << 31 ) || !trace1d_metrics_ok( p.Nx ) ) return hipErrorInvalidValue;
+    uint32_t threads = 256;
+    while ( threads < 1024 && nodes > uint64_t( threads ) * uint64_t( n_cu ) ) threads *= 2;
+    bool pipe = false;
+    uint64_t c = poly_chunk_plan( p.Nx, sizeof(double), 1u << 20, std::min<size_t>( lds_cap, 160 * 1024 ), &pipe );
+    if ( p.n < c ) c = p.n > 0 ? p.n : 1;
+    p.chunk = uint32_t( c ); p.pipe = pipe ? 1u : 0u;
+    p.n_tasks = uint32_t( ( nodes + WAVE - 1 ) / WAVE );
+    *tasks = p.n_tasks;
+    const size_t lds = ( pipe ? 2 : 1 ) * size_t( c ) * p.stride_q * sizeof(double);
+    const uint32_t grid = uint32_t( ( nodes + threads - 1 ) / threads );
+    return ( p.Nx & ( p.Nx - 1 ) ) == 0 ? launch_kernel( trace1d_metrics_kernel<true>, grid, int( threads ), lds, p, st )
+                                        : launch_kernel( trace1d_metrics_kernel<false>, grid, int( threads ), lds, p, st );
 }
 
 hipError_t launch_trace1d( const trace1_params &p_in, int variant, const launch_shape &s, int n_cu, hipStream_t st )
