@@ -736,7 +736,7 @@ def main():
     e64 = h64 = None
     if args.only in ("fp64", "both"):
         r64, e64, h64, s64 = landau3d_form(c5, nufi.FP64, args.steps, args.warmup, args.autotune, FLOPS_3D,
-                                           "trace3d_xm_fast_kernel")
+                                           "trace3d_zcell_kernel")
         l3["fp64"] = r64
         progress(f"3D Landau FP64: {r64['time_to_T_s']:.2f} s to T, {r64['ms_per_step']:.1f} ms per step n=80")
         if with_cpu and args.case == "all":
@@ -780,7 +780,7 @@ def main():
         "peak_measured_note": "FMA-chain probe on the box (profiles/peaks_mi355x.md); peak stays the published figure",
     })
     if prim_prec == "fp64":
-        ex = read_executed_flops("trace3d_landau3d_pmc.json", "trace3d_xm_fast_kernel", prim["char_steps_per_step"])
+        ex = read_executed_flops("trace3d_landau3d_pmc.json", "trace3d_zcell_kernel", prim["char_steps_per_step"])
         if ex is not None:
             roofline["executed_flops_per_char_step"] = ex
             roofline["achieved_executed"] = ex * prim["char_steps_per_step"] / (roofline["avg_launch_ms"] * 1e-3) / 1e12

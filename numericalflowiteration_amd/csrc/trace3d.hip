@@ -6,6 +6,9 @@
 // splines.hpp:144-172); kick u,v,w.  After the loop a final drift and
 // half-kick with slice 0, and f0 at the foot.
 //
+// FP64 rho and metrics of grids whose z-cell window fits the LDS run in
+// trace3d_zcell.hip; launch_trace3d hands rho over.  Here:
+//
 // The workgroup streams coefficient slices through LDS (one slice is
 // (Nx+3)(Ny+3)(Nz+3) reals: 6859 = 54.9 KB FP64 at 16^3) and every node
 // gathers its 4x4x4 window from LDS.  The fast FP64 rho kernel lays a wave's
