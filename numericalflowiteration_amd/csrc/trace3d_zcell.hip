@@ -44,6 +44,7 @@
 #include "device_common.hpp"
 #include "internal.hpp"
 #include "step3d.hpp"
+#include "zcell_index.hpp"
 
 #include <stddef.h>
 #include <type_traits>
@@ -392,14 +393,7 @@ void trace3d_zcell_kernel( trace3_params p )
             double z = still ? sz_[r] : fma( -cdz, vw[r], sz_[r] );
             if ( !MASK ) z = fma( -Nd[2], floor( z * iN[2] ), z );
             sz_[r] = z;
-            int d = int( floor( z ) ) - zb;
-            if ( MASK ) d &= Nzi - 1;
-            else
-            {
-                d = d < 0 ? d + Nzi : d;
-                d = d >= Nzi ? d - Nzi : d;
-            }
-            rel[r] = uint32_t( d );
+            rel[r] = zc_rel<MASK>( int( floor( z ) ), zb, Nzi );
             worst = worst > rel[r] ? worst : rel[r];
         }
         auto node = [&]( double &x, double &y, double z, double &u, double &v, double &w, uint32_t rl, bool local )
@@ -431,9 +425,9 @@ void trace3d_zcell_kernel( trace3_params p )
             }
             else
             {
-                uint32_t cell = uint32_t( zb ) + rl;
-                if ( cell >= p.Nz ) cell -= p.Nz;
-                const double *h = p.hist + size_t( m ) * p.st + size_t( cell ) * plane + uint32_t( j ) * sy + uint32_t( i );
+                // global memory: whatever the position, a cell of the slice
+                const double *h = p.hist + size_t( m ) * p.st + size_t( zc_cell( zb, rl, p.Nz ) ) * plane +
+                                  zc_held( j, uint32_t( Nyi ) ) * sy + zc_held( i, Nx );
                 zc_gradient( [&]( int idx, double c[4] )
                 {
                     const double *q = h + uint32_t( idx >> 2 ) * sy + uint32_t( idx & 3 );

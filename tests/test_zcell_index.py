@@ -1,0 +1,64 @@
+"""Cell numbers of the z-cell 3D trace (csrc/zcell_index.hpp), compiled by the
+host compiler: what the kernel reads from the global history stays inside the
+slice for every integer a position may leave as its cell (positions too large to
+be wrapped exactly leave any, up to the saturated ends of int; NaN leaves 0),
+and is the periodic cell for every position within a period of the window."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "numericalflowiteration_amd", "csrc")
+
+SOURCE = r"""
+#include "zcell_index.hpp"
+#include <cstdio>
+#include <climits>
+using namespace nufi_impl;
+
+template <bool MASK> int grid( int N )
+{
+    const long long wild[] = { INT_MIN, INT_MIN + 1, -2147479552LL, -4096, -1000003, 1000003, 4096, 123456789,
+                               INT_MAX - 1, INT_MAX, -N, -N - 1, 2 * N, 2 * N + 1, 0 };
+    for ( int zb = 0; zb < N; ++zb )
+    {
+        for ( int c = -1; c <= N; ++c )            // what the wrap leaves: one rounding past either end
+        {
+            const uint32_t rel = zc_rel<MASK>( c, zb, N );
+            const int want = ( c + N ) % N;
+            if ( rel >= uint32_t( N ) || int( zc_cell( zb, rel, N ) ) != want ) return std::printf( "cell %d of %d\n", c, N ), 1;
+        }
+        for ( long long w : wild )
+        {
+            const uint32_t rel = zc_rel<MASK>( int( w ), zb, N );
+            if ( zc_cell( zb, rel, N ) >= uint32_t( N ) ) return std::printf( "wild %lld of %d from %d\n", w, N, zb ), 1;
+        }
+    }
+    for ( int i = 0; i < N; ++i ) if ( zc_held( i, N ) != uint32_t( i ) ) return std::printf( "held %d of %d\n", i, N ), 1;
+    for ( long long w : wild ) if ( zc_held( int( w ), N ) >= uint32_t( N ) ) return std::printf( "held %lld of %d\n", w, N ), 1;
+    return 0;
+}
+
+int main()
+{
+    int bad = 0;
+    for ( int N = 1; N <= 40; ++N ) bad += grid<false>( N );
+    for ( int N = 1; N <= 64; N *= 2 ) bad += grid<true>( N );
+    return bad ? 1 : 0;
+}
+"""
+
+
+def test_cells_stay_inside_the_slice(tmp_path):
+    src = tmp_path / "t.cpp"
+    src.write_text(SOURCE)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-fwrapv", "-I", CSRC, str(src), "-o", str(tmp_path / "t")],
+                   check=True)
+    r = subprocess.run([str(tmp_path / "t")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
+
+
+def test_the_kernel_reads_the_global_history_through_them():
+    text = open(os.path.join(CSRC, "trace3d_zcell.hip")).read()
+    reads = [ln for ln in text.splitlines() if "const double *h = p.hist" in ln]
+    assert len(reads) == 1 and "zc_cell(" in reads[0]
+    assert "zc_held( j" in text and "zc_held( i" in text
