@@ -33,6 +33,7 @@
 #include <algorithm>
 
 #include "device_common.hpp"
+#include "cell_index.hpp"
 #include "internal.hpp"
 #include "step1d.hpp"
 #include "strict1d.hpp"
@@ -403,7 +404,7 @@ void trace1d_metrics_kernel( trace1_params p )
     {
         const double *Q = p.qhist + size_t( p.n ) * sq;
         double t;
-        const int i = wrap_locate( s, Nxd, invNx, t );
+        const int i = table_cell( wrap_locate( s, Nxd, invNx, t ), int( p.Nx ) );      // global memory: wherever the grid lies
         const double2 q01 = reinterpret_cast<const double2*>( Q )[ i + 1 ];
         u = fma( 0.5 * p.kick, fma( fma( Q[ q2 + ( i + 1 ) ], t, q01.y ), t, q01.x ), u );
         auto steps = [&]( const double *C, int mlo, int hi, int )

@@ -44,7 +44,7 @@
 #include "device_common.hpp"
 #include "internal.hpp"
 #include "step3d.hpp"
-#include "zcell_index.hpp"
+#include "cell_index.hpp"
 
 #include <stddef.h>
 #include <type_traits>

@@ -1,8 +1,9 @@
-"""Cell numbers of the z-cell 3D trace (csrc/zcell_index.hpp), compiled by the
-host compiler: what the kernel reads from the global history stays inside the
-slice for every integer a position may leave as its cell (positions too large to
-be wrapped exactly leave any, up to the saturated ends of int; NaN leaves 0),
-and is the periodic cell for every position within a period of the window."""
+"""Cell numbers of the z-cell 3D trace and of the 1D metrics' first half kick
+(csrc/cell_index.hpp), compiled by the host compiler: what the kernels read from
+global memory stays inside the slice or table for every integer a position may
+leave as its cell (positions too large to be wrapped exactly leave any, up to the
+saturated ends of int; NaN leaves 0), and is the periodic cell for every position
+within a period."""
 import os
 import subprocess
 
@@ -10,7 +11,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "numericalflowiteration_amd", "csrc")
 
 SOURCE = r"""
-#include "zcell_index.hpp"
+#include "cell_index.hpp"
 #include <cstdio>
 #include <climits>
 using namespace nufi_impl;
@@ -35,6 +36,9 @@ template <bool MASK> int grid( int N )
     }
     for ( int i = 0; i < N; ++i ) if ( zc_held( i, N ) != uint32_t( i ) ) return std::printf( "held %d of %d\n", i, N ), 1;
     for ( long long w : wild ) if ( zc_held( int( w ), N ) >= uint32_t( N ) ) return std::printf( "held %lld of %d\n", w, N ), 1;
+    for ( int i = -1; i <= N; ++i ) if ( table_cell( i, N ) != i ) return std::printf( "table %d of %d\n", i, N ), 1;
+    for ( long long w : wild )
+        if ( table_cell( int( w ), N ) < -1 || table_cell( int( w ), N ) > N ) return std::printf( "table %lld of %d\n", w, N ), 1;
     return 0;
 }
 
@@ -48,7 +52,7 @@ int main()
 """
 
 
-def test_cells_stay_inside_the_slice(tmp_path):
+def test_cells_stay_inside(tmp_path):
     src = tmp_path / "t.cpp"
     src.write_text(SOURCE)
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-fwrapv", "-I", CSRC, str(src), "-o", str(tmp_path / "t")],
@@ -57,8 +61,12 @@ def test_cells_stay_inside_the_slice(tmp_path):
     assert r.returncode == 0, r.stdout
 
 
-def test_the_kernel_reads_the_global_history_through_them():
+def test_the_kernels_read_global_memory_through_them():
     text = open(os.path.join(CSRC, "trace3d_zcell.hip")).read()
     reads = [ln for ln in text.splitlines() if "const double *h = p.hist" in ln]
     assert len(reads) == 1 and "zc_cell(" in reads[0]
     assert "zc_held( j" in text and "zc_held( i" in text
+
+    text = open(os.path.join(CSRC, "trace1d.hip")).read()
+    body = text[text.index("void trace1d_metrics_kernel"):]
+    assert "table_cell( wrap_locate(" in body[:body.index("poly_ready_pipeline")]
