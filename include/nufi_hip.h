@@ -220,6 +220,18 @@ int nufi_get_launch_shape(nufi_ctx *ctx, int *block, int *nodes_per_thread, int 
 int nufi_autotune(nufi_ctx *ctx, uint64_t n_probe, int repeats, int *block, int *nodes_per_thread,
                   int *chunk, double *best_ms);
 
+/*
+ * How the last 3D FP64 trace (rho over all nodes, or metrics) of ctx ran; waits
+ * for the stream.  out[0]: 1 where the z-cell trace takes the grid (the rest is 0
+ * otherwise); out[1]: 1 if the history had it trace from whole slices instead;
+ * out[2]: the bound on how far nodes get apart that was decided by, in 1/65536
+ * cells; out[3]: what nodes outside their window were found to cost, in 1/65536
+ * of a workgroup's trace (0 where the bound settled it); out[4]: workgroups
+ * redone from whole slices; out[5]: workgroups.  Calls of fewer than 16 slices
+ * decide nothing and leave out[1..3] as they were.
+ */
+int nufi_trace3d_route(nufi_ctx *ctx, uint64_t out[6]);
+
 /* ---- timing of the trace kernel ---------------------------------------- */
 /*
  * When enabled, every trace-kernel launch is bracketed by HIP events on the

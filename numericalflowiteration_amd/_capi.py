@@ -74,6 +74,7 @@ SIGNATURES = {
                              _dp]),
     "nufi_set_timing": (_int, [_vp, _int]),
     "nufi_trace_timing": (_int, [_vp, ctypes.POINTER(_u64), _dp, _dp]),
+    "nufi_trace3d_route": (_int, [_vp, ctypes.POINTER(_u64)]),
     "nufi_adjoint_grad": (_int, [_vp, _dp, _int, _dp]),
     "nufi_rho3d_noalloc": (_int, [_cp, _u64, _vp, _u64, _vp, _vp]),
     "nufi_batch_create": (_int, [_cp, _u64, _int, _int, _int, ctypes.POINTER(_vp)]),

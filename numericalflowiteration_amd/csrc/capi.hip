@@ -39,7 +39,7 @@ struct nufi_ctx
     uint32_t st32 = 0;         // hist32 slice stride: st rounded up to 4 floats
     uint64_t n_space = 0, n_vel = 0, n_nodes = 0;
     uint32_t wpx = 0;          // wave-task partials per spatial point (strict 1D, 3D)
-    uint32_t ppx = 0;          // x-major partials per spatial point (fast; 1D FP32C)
+    uint32_t ppx = 0;          // x-major partials per spatial point (fast; 1D FP32C); 3D: the window kernel's
     uint32_t vgroup = 0;       // 3D x-major: velocities per partial
     zcell_plan zc {};          // 3D fast FP64 (rho and metrics): the z-cell kernel's layout, zc.ok where it runs
     int field_ok = 0;          // 1: one-workgroup field solve; 2: the multi-workgroup one; 0: none
@@ -131,7 +131,7 @@ void free_all( nufi_ctx *c )
     void *ptrs[] = { c->hist, c->dhist, c->qhist, c->qhist32, c->hist32, c->partials, c->rho, c->energies,
                      c->values, c->scratch_slice, c->metrics, c->mpartials, c->energy_tmp,
                      c->rho_hist, c->lambda, c->gvec, c->grad_part, c->grad, c->tw_x, c->tw_y, c->tw_z,
-                     c->mult_step, c->mult_pois, c->mult_fit, c->ewt, c->samp, c->lw0, c->lw1, c->lpart, c->zc.marks };
+                     c->mult_step, c->mult_pois, c->mult_fit, c->ewt, c->samp, c->lw0, c->lw1, c->lpart, c->zc.marks, c->zc.route };
     if ( c->run_graph ) (void)hipGraphExecDestroy( c->run_graph );
     c->run_graph = nullptr;
     for ( void *p : ptrs ) if ( p ) (void)hipFree( p );
@@ -203,7 +203,14 @@ int build_tables( nufi_ctx *c )
 uint32_t rho_ppx( const nufi_ctx *c )
 {
     const bool xm = c->variant == TRACE_FAST || ( c->dim == 1 && c->variant == TRACE_FP32C );
-    return xm ? c->ppx : c->wpx;
+    return xm ? ( c->zc.ok ? c->zc.ppx : c->ppx ) : c->wpx;
+}
+
+// and those of the window kernel where step n may take it
+partial_alt rho_alt( const nufi_ctx *c, uint64_t n )
+{
+    if ( c->dim != 3 || c->variant != TRACE_FAST ) return partial_alt {};
+    return partial_alt { zcell_window( c->zc, n, c->conf.Nx, c->conf.Ny, c->conf.Nz ), c->ppx };
 }
 
 // The chunk a rho launch of shape s uses and its LDS: 1D x-major launches
@@ -513,7 +520,6 @@ int nufi_create( const nufi_config *conf, const nufi_config *conf_metrics, int o
         c->vgroup = xm3_vgroup( c->n_space, c->n_vel );
         c->ppx = uint32_t( ( c->n_vel + c->vgroup - 1 ) / c->vgroup );
         c->zc = plan_zcell( *conf );
-        if ( c->zc.ok ) c->ppx = c->zc.ppx;
     }
     c->field_ok = field_supported( c->dim, uint32_t( conf->Nx ), c->dim == 3 ? uint32_t( conf->Ny ) : 1u,
                                    c->dim == 3 ? uint32_t( conf->Nz ) : 1u );
@@ -537,7 +543,7 @@ int nufi_create( const nufi_config *conf, const nufi_config *conf_metrics, int o
     c->st32 = ( c->st + 3u ) & ~3u;
     if ( precision == NUFI_FP32C && c->dim == 3 && ( rc = dev_alloc( c, &c->hist32, slices * c->st32 + 8, "FP32 history" ) ) )
         return bail( rc );
-    if ( ( rc = dev_alloc( c, &c->partials, c->n_space * std::max( c->wpx, c->ppx ), "partials" ) ) ) return bail( rc );
+    if ( ( rc = dev_alloc( c, &c->partials, c->n_space * std::max( { c->wpx, c->ppx, c->zc.ppx } ), "partials" ) ) ) return bail( rc );
     if ( ( rc = dev_alloc( c, &c->rho, c->n_space, "rho" ) ) ) return bail( rc );
     if ( ( rc = dev_alloc( c, &c->values, c->n_space, "values" ) ) ) return bail( rc );
     if ( ( rc = dev_alloc( c, &c->energies, slices, "energies" ) ) ) return bail( rc );
@@ -550,6 +556,7 @@ int nufi_create( const nufi_config *conf, const nufi_config *conf_metrics, int o
     c->m_nodes = c->m_space * c->m_vel;
     c->m_wpx = uint32_t( ( c->m_vel + 63 ) / 64 );
     if ( c->zc.ok && ( rc = dev_alloc( c, &c->zc.marks, zcell_workgroups( *conf, c->zc, nullptr ), "window marks" ) ) ) return bail( rc );
+    if ( c->zc.ok && ( rc = dev_alloc( c, &c->zc.route, 1, "trace route" ) ) ) return bail( rc );
     const size_t m_waves = std::max<size_t>( c->m_space * c->m_wpx, c->zc.ok ? zcell_metric_waves( *conf, c->zc ) : 0 );
     if ( ( rc = dev_alloc( c, &c->mpartials, 4 * m_waves, "metric partials" ) ) ) return bail( rc );
     if ( c->field_ok && ( rc = build_tables( c ) ) ) return bail( rc );
@@ -609,7 +616,7 @@ int nufi_compute_rho( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_end 
     if ( rc ) return rc;
     hipError_t e = launch_reduce_partials( c->partials, rho_ppx( c ), rho_weight( c ), uint32_t( first ), uint32_t( count ),
                                            uint32_t( c->n_space ), field_sum_group( c->n_space, c->precision == NUFI_FP32C ),
-                                           c->rho, c->stream );
+                                           c->rho, c->stream, rho_alt( c, n ) );
     if ( e != hipSuccess ) return hip_fail( c, e, "reduce launch" );
     return NUFI_OK;
 }
@@ -657,6 +664,7 @@ int nufi_compute_metrics( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_
         return fail( c, NUFI_ERR_UNSUPPORTED, "compute_metrics: one FP64 slice of this grid exceeds the LDS" );
     HIP_TRY( c, hipSetDevice( c->device ) );
     uint64_t tasks = 0;
+    partial_alt alt {};
     if ( q_begin < q_end )
     {
         const uint64_t l0 = q_begin / c->m_vel, l1 = ( q_end - 1 ) / c->m_vel;
@@ -702,14 +710,25 @@ int nufi_compute_metrics( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_
             {
                 uint32_t waves = 0;
                 p.n_count = uint32_t( l1 - l0 + 1 ); p.zc = c->zc;
+                // where the route leaves the z-cells: small slices, cheap to stage, in wave
+                // tasks (11 x 13 x 9, mixing by 2: 1.9 ms, by trace3d_zslice_kernel 2.5),
+                // others by that (16^3 116 / 73 ms)
+                const bool wave_tasks = zcell_routed( c->zc, n, g.Nz ) && c->st <= 5120;
+                p.zc.flag_mark = wave_tasks ? 0u : 1u;
                 e = launch_trace3d_zcell( p, &waves, c->stream );
+                if ( e == hipSuccess && wave_tasks )
+                {
+                    p.run_if = &c->zc.route->window;
+                    alt = partial_alt { p.run_if, uint32_t( tasks ) };
+                    e = launch_trace3d( p, variant, launch_shape { 256, 1, 1 }, c->stream );
+                }
                 tasks = waves;
             }
             else e = launch_trace3d( p, variant, launch_shape { 256, 1, 1 }, c->stream );
         }
         if ( e != hipSuccess ) return hip_fail( c, e, "metrics trace launch" );
     }
-    hipError_t e = launch_reduce_metrics( c->mpartials, uint32_t( tasks ), c->metrics, c->stream );
+    hipError_t e = launch_reduce_metrics( c->mpartials, uint32_t( tasks ), c->metrics, c->stream, alt );
     if ( e != hipSuccess ) return hip_fail( c, e, "metrics reduce launch" );
     return NUFI_OK;
 }
@@ -745,13 +764,14 @@ static int step_async( nufi_ctx *c, uint64_t n, double *rho_out )
     field_params f = base_field( c );
     f.mode = FIELD_STEP;
     f.partials = c->partials;
-    if ( uint64_t( f.wpx ) * c->n_space > ( uint64_t( 1 ) << 16 ) )
+    f.alt = rho_alt( c, n );
+    if ( uint64_t( f.alt.sel ? std::max( f.wpx, f.alt.count ) : f.wpx ) * c->n_space > ( uint64_t( 1 ) << 16 ) )
     {
         // many partials (3D): one thread per point over many workgroups sums them
         // in the same order, and the single field workgroup starts from rho
         double *dst = rho_out ? rho_out : c->rho;
         hipError_t e = launch_reduce_partials( c->partials, f.wpx, f.weight, 0, uint32_t( c->n_space ),
-                                               uint32_t( c->n_space ), f.sum_group, dst, c->stream );
+                                               uint32_t( c->n_space ), f.sum_group, dst, c->stream, f.alt );
         if ( e != hipSuccess ) return hip_fail( c, e, "reduce launch" );
         f.partials = nullptr;
         f.values = dst;
@@ -1245,6 +1265,23 @@ int nufi_trace_timing( nufi_ctx *c, uint64_t *launches, double *kernel_ms, doubl
     if ( launches ) *launches = c->launches;
     if ( kernel_ms ) *kernel_ms = ms;
     if ( char_steps ) *char_steps = c->csteps;
+    return NUFI_OK;
+}
+
+int nufi_trace3d_route( nufi_ctx *c, uint64_t out[6] )
+{
+    if ( c == nullptr || out == nullptr ) return NUFI_ERR_INVALID;
+    for ( int k = 0; k < 6; ++k ) out[k] = 0;
+    if ( !c->zc.ok ) return NUFI_OK;
+    HIP_TRY( c, hipSetDevice( c->device ) );
+    HIP_TRY( c, hipStreamSynchronize( c->stream ) );
+    zcell_route r {};
+    std::vector<uint32_t> marks( zcell_workgroups( c->conf, c->zc, nullptr ) );
+    HIP_TRY( c, hipMemcpy( &r, c->zc.route, sizeof(r), hipMemcpyDeviceToHost ) );
+    HIP_TRY( c, hipMemcpy( marks.data(), c->zc.marks, marks.size() * sizeof(uint32_t), hipMemcpyDeviceToHost ) );
+    out[0] = 1; out[1] = r.window; out[2] = r.last_spread; out[3] = r.last_cost;
+    for ( uint32_t m : marks ) out[4] += m;
+    out[5] = marks.size();
     return NUFI_OK;
 }
 

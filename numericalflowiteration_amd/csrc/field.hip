@@ -194,10 +194,10 @@ __device__ __forceinline__ void field_body( const field_params &p, double2 *lds2
     // 1. rho (or the nodal values) into A
     if ( p.mode == FIELD_STEP && p.partials != nullptr )
     {
-        const uint32_t G = p.sum_group, part = threadIdx.x & ( G - 1 );
+        const uint32_t G = p.sum_group, part = threadIdx.x & ( G - 1 ), wpx = partial_count( p.wpx, p.alt );
         for ( uint32_t i = threadIdx.x / G; i < N; i += FIELD_BLOCK / G )
         {
-            const double v = p.weight * sum_partials( p.partials, p.wpx, N, i, part, G );
+            const double v = p.weight * sum_partials( p.partials, wpx, N, i, part, G );
             if ( part != 0 ) continue;
             if ( p.rho_out ) p.rho_out[i] = v;
             A[i] = make_double2( v, 0.0 );
@@ -292,12 +292,13 @@ void field_batch_kernel( const batch_field *__restrict__ runs, uint64_t n )
 }
 
 __global__ __launch_bounds__( 64 ) void reduce_partials_kernel( const double *partials, uint32_t wpx, double weight,
-                                        uint32_t first, uint32_t count, uint32_t n_space, uint32_t G, double *rho )
+                                        uint32_t first, uint32_t count, uint32_t n_space, uint32_t G, double *rho,
+                                        partial_alt alt )
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, i = t / G, part = t & ( G - 1 );
     if ( i >= n_space ) return;
     double v = 0.0;
-    if ( i >= first && i < first + count ) v = weight * sum_partials( partials, wpx, n_space, i, part, G );
+    if ( i >= first && i < first + count ) v = weight * sum_partials( partials, partial_count( wpx, alt ), n_space, i, part, G );
     if ( part == 0 ) rho[i] = v;
 }
 
@@ -324,8 +325,9 @@ __global__ void slice_tables_kernel( int dim, const double *slice, uint32_t len,
 
 // metrics[k] = sum over tasks of partials[4 g + k], compensated, fixed order
 __global__ __launch_bounds__( 256 )
-void reduce_metrics_kernel( const double *partials, uint32_t n_tasks, double *metrics )
+void reduce_metrics_kernel( const double *partials, uint32_t n_tasks_, double *metrics, partial_alt alt )
 {
+    const uint32_t n_tasks = partial_count( n_tasks_, alt );
     __shared__ double red_s[4][4], red_c[4][4];
     csum acc[4] = { { 0, 0 }, { 0, 0 }, { 0, 0 }, { 0, 0 } };
     for ( uint32_t g = threadIdx.x; g < n_tasks; g += 256 )
@@ -349,9 +351,9 @@ void reduce_metrics_kernel( const double *partials, uint32_t n_tasks, double *me
 
 } // namespace
 
-hipError_t launch_reduce_metrics( const double *partials, uint32_t n_tasks, double *metrics, hipStream_t st )
+hipError_t launch_reduce_metrics( const double *partials, uint32_t n_tasks, double *metrics, hipStream_t st, partial_alt alt )
 {
-    hipLaunchKernelGGL( reduce_metrics_kernel, dim3( 1 ), dim3( 256 ), 0, st, partials, n_tasks, metrics );
+    hipLaunchKernelGGL( reduce_metrics_kernel, dim3( 1 ), dim3( 256 ), 0, st, partials, n_tasks, metrics, alt );
     return hipGetLastError();
 }
 
@@ -427,11 +429,11 @@ size_t field_batch_lds_bytes( uint32_t max_N, int *tw_lds )
 
 hipError_t launch_reduce_partials( const double *partials, uint32_t wpx, double weight,
                                    uint32_t first, uint32_t count, uint32_t n_space, uint32_t G,
-                                   double *rho, hipStream_t st )
+                                   double *rho, hipStream_t st, partial_alt alt )
 {
     const uint32_t block = 64, grid = ( n_space * G + block - 1 ) / block;     // a group per point, many CUs
     hipLaunchKernelGGL( reduce_partials_kernel, dim3( grid ), dim3( block ), 0, st,
-                        partials, wpx, weight, first, count, n_space, G, rho );
+                        partials, wpx, weight, first, count, n_space, G, rho, alt );
     return hipGetLastError();
 }
 

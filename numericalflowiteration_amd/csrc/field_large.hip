@@ -42,7 +42,7 @@ __global__ __launch_bounds__( LB ) void large_load_kernel( field_params p, doubl
 {
     const uint32_t i = blockIdx.x * LB + threadIdx.x;
     if ( i >= p.N ) return;
-    const double v = ( p.mode == FIELD_STEP && p.partials != nullptr ) ? p.weight * sum_partials_l( p.partials, p.wpx, p.N, i )
+    const double v = ( p.mode == FIELD_STEP && p.partials != nullptr ) ? p.weight * sum_partials_l( p.partials, partial_count( p.wpx, p.alt ), p.N, i )
                                                                       : p.values[i];
     if ( p.rho_out ) p.rho_out[i] = v;
     W[i] = make_double2( v, 0.0 );

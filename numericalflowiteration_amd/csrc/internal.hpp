@@ -106,6 +106,16 @@ struct zcell_consts          // per axis: points, their inverse, drift in cells 
 {
     double N[3], iN[3], cd[3], kick[3], kickh[3];
 };
+// Which kernel traces a call (trace3d_zcell.hip), decided on the device by the
+// history the call reads: one per context, written by each call before it is read.
+struct zcell_route
+{
+    uint32_t window;         // 1: whole slices (trace3d_zslice_kernel or the window kernel), not z-cells
+    uint32_t scout;          // 1: the bound left it open, scouts decide
+    uint32_t arrived[2];     // workgroups of the two deciding kernels that are done
+    unsigned long long spread, cost;           // their sums (integers: any order gives the same)
+    unsigned long long last_spread, last_cost; // of the last call, for reports
+};
 struct zcell_plan
 {
     bool ok;
@@ -116,6 +126,8 @@ struct zcell_plan
                                                // group blocks a w, first z plane
     uint32_t inv_nx;         // ceil(2^20 / Nx)
     uint32_t *marks;         // per workgroup: 1 where the window did not hold its nodes
+    uint32_t flag_mark;      // per launch: the mark of a workgroup that the route takes off the z-cell kernel
+    zcell_route *route;
     zcell_consts k;
 };
 inline size_t zcell_lds( uint32_t nzc, uint32_t cols, uint32_t szp )
@@ -162,6 +174,7 @@ struct trace3_params
     double kick72[3], kick72h[3]; // fast FP64: -dt d_inv / 72 per axis (72-scaled gradient), and half of it
     float f32_p0[3], f32_w0[3];   // FP32C: offsets of the position and velocity hi parts per axis
     zcell_plan zc;                // fast FP64: the z-cell kernel's layout (zc.ok), else the window kernel
+    const uint32_t *run_if;       // nullable: the launch traces where this is not 0
     nufi_f0 f0;
 };
 
@@ -247,6 +260,25 @@ size_t zcell_metric_waves( const nufi_config &g, const zcell_plan &z );
 // workgroups (and their waves) of a whole-grid launch, at most ZCELL_MARKS; a mark each
 size_t zcell_workgroups( const nufi_config &g, const zcell_plan &z, uint32_t *waves );
 hipError_t launch_trace3d_zcell( const trace3_params &p, uint32_t *tasks, hipStream_t st );
+// Whether a call of n slices lets the device choose between z-cells and whole
+// slices (zc.route->window).  Below ZCELL_ROUTE_MIN slices only kicks that differ
+// by more than 0.04 cells a step and step take nodes out of a window (a potential
+// of twice the thermal energy at 16^3), and the deciding launches (6 us) are up to a
+// tenth of a call.
+constexpr uint64_t ZCELL_ROUTE_MIN = 16;
+inline bool zcell_routed( const zcell_plan &z, uint64_t n, uint64_t Nz )
+{
+    return z.ok && z.route != nullptr && z.nzc < Nz && n >= ZCELL_ROUTE_MIN;
+}
+// The flag by which the window kernel traces rho in the z-cell workgroups' place,
+// null where it never does.  At 16^3 its compiled strides and eight nodes a lane
+// beat trace3d_zslice_kernel (n = 60, 24^3 velocities, mixing by 0.4: 47 against 55 ms);
+// elsewhere that one is as fast or faster (20^3 143 / 136, 20 x 18 x 20 32.7 / 30.4,
+// 11 x 13 x 9 3.1 / 2.3, 8^3 1.40 / 1.09, 24 x 20 x 12 25.5 / 26.4) and saves a launch.
+inline const uint32_t *zcell_window( const zcell_plan &z, uint64_t n, uint64_t Nx, uint64_t Ny, uint64_t Nz )
+{
+    return Nx == 16 && Ny == 16 && Nz == 16 && zcell_routed( z, n, Nz ) ? &z.route->window : nullptr;
+}
 size_t trace1d_slice_elems( const trace1_params &p, int variant );
 hipError_t launch_trace1d_batch( const batch_run *runs, const uint32_t *wg_run, uint32_t n_wg, uint64_t n,
                                  int variant, const launch_shape &s, size_t lds, hipStream_t st );
@@ -341,6 +373,18 @@ enum field_mode : int
     FIELD_FIT     = 2  // nodal values -> slice
 };
 
+// Another count of partials per point (or of metric partials), in force where
+// *sel is not 0; sel may be null.
+struct partial_alt
+{
+    const uint32_t *sel;
+    uint32_t count;
+};
+__device__ __forceinline__ uint32_t partial_count( uint32_t count, const partial_alt &alt )
+{
+    return alt.sel != nullptr && *alt.sel != 0 ? alt.count : count;
+}
+
 struct field_params
 {
     int      dim, order, mode;
@@ -350,6 +394,7 @@ struct field_params
     uint32_t sum_group;          // threads that share a point's partial sums (field_sum_group)
     const double *partials;      // FIELD_STEP: partials (nullable -> use values)
     uint32_t wpx;
+    partial_alt alt;
     double   weight;             // -dv multiplier applied to partial sums
     double  *values;             // rho / phi (FIELD_POISSON in/out, FIELD_FIT in)
     double  *rho_out;            // optional copy of rho
@@ -399,13 +444,14 @@ size_t field_lds_bytes( const field_params &p );
 int field_supported( int dim, uint32_t Nx, uint32_t Ny, uint32_t Nz );
 
 // metrics[k] = sum_g partials[4*g + k] in a fixed order (one workgroup).
-hipError_t launch_reduce_metrics( const double *partials, uint32_t n_tasks, double *metrics, hipStream_t st );
+hipError_t launch_reduce_metrics( const double *partials, uint32_t n_tasks, double *metrics, hipStream_t st,
+                                  partial_alt alt = partial_alt {} );
 
 // Sum of the partials into rho[ix] = weight * sum_j partials[j*n_space + ix]
 // for ix in [first, first+count), zero elsewhere (n_space entries).
 hipError_t launch_reduce_partials( const double *partials, uint32_t wpx, double weight,
                                    uint32_t first, uint32_t count, uint32_t n_space, uint32_t G,
-                                   double *rho, hipStream_t st );       // G: field_sum_group
+                                   double *rho, hipStream_t st, partial_alt alt = partial_alt {} );       // G: field_sum_group
 // The 1D FP32C trace carries its velocities in cells per step (w = dt dx_inv
 // u): its FP32 kick-polynomial tables are scaled in FP64 by the kick
 // -dt dx_inv / 2 times dt dx_inv before their one rounding.

@@ -26,10 +26,12 @@ namespace
 constexpr size_t SCRATCH_DOUBLES = NUFI_NOALLOC_SCRATCH_BYTES / sizeof(double);
 static __device__ __align__( 256 ) double scratch[SCRATCH_DOUBLES];
 static __device__ uint32_t marks[nufi_impl::ZCELL_MARKS];          // the z-cell trace's window marks
+static __device__ nufi_impl::zcell_route route;                    // and route
 
 constexpr int MAX_DEVICES = 64;
 double *g_scratch[MAX_DEVICES] = {};
 uint32_t *g_marks[MAX_DEVICES] = {};
+nufi_impl::zcell_route *g_route[MAX_DEVICES] = {};
 std::mutex g_scratch_mu;
 
 int fail( int code, const std::string &msg )
@@ -38,8 +40,8 @@ int fail( int code, const std::string &msg )
     return code;
 }
 
-// The current device's copies of `scratch` and `marks` (looked up once per device).
-int device_scratch( double **out, uint32_t **out_marks )
+// The current device's copies of `scratch`, `marks` and `route` (looked up once per device).
+int device_scratch( double **out, uint32_t **out_marks, nufi_impl::zcell_route **out_route )
 {
     int dev = 0;
     hipError_t e = hipGetDevice( &dev );
@@ -56,11 +58,17 @@ int device_scratch( double **out, uint32_t **out_marks )
         e = hipGetSymbolAddress( &q, HIP_SYMBOL( marks ) );
         if ( e != hipSuccess || q == nullptr )
             return fail( NUFI_ERR_DEVICE, std::string( "rho3d_noalloc: hipGetSymbolAddress: " ) + hipGetErrorString( e ) );
+        void *r = nullptr;
+        e = hipGetSymbolAddress( &r, HIP_SYMBOL( route ) );
+        if ( e != hipSuccess || r == nullptr )
+            return fail( NUFI_ERR_DEVICE, std::string( "rho3d_noalloc: hipGetSymbolAddress: " ) + hipGetErrorString( e ) );
+        g_route[dev] = static_cast<nufi_impl::zcell_route*>( r );
         g_scratch[dev] = static_cast<double*>( p );
         g_marks[dev] = static_cast<uint32_t*>( q );
     }
     *out = g_scratch[dev];
     *out_marks = g_marks[dev];
+    *out_route = g_route[dev];
     return NUFI_OK;
 }
 
@@ -101,7 +109,8 @@ extern "C" int nufi_rho3d_noalloc( const nufi_config *conf, uint64_t n, const do
     }
     double *part = nullptr;
     uint32_t *mk = nullptr;
-    int rc = device_scratch( &part, &mk );
+    zcell_route *rt = nullptr;
+    int rc = device_scratch( &part, &mk, &rt );
     if ( rc ) return rc;
 
     trace3_params p {};
@@ -113,14 +122,15 @@ extern "C" int nufi_rho3d_noalloc( const nufi_config *conf, uint64_t n, const do
     p.sy = uint32_t( sy ); p.sz = uint32_t( sz ); p.st = uint32_t( st ); p.st32 = uint32_t( ( st + 3 ) & ~uint64_t( 3 ) );
     p.wpx = uint32_t( wpx );
     p.l_first = 0; p.n_tasks = uint32_t( n_space * wpx ); p.n_count = uint32_t( n_space );
-    p.vgroup = vgroup; p.ppx = uint32_t( ppx ); p.zc = zc; p.zc.marks = mk;
+    p.vgroup = vgroup; p.ppx = uint32_t( ppw ); p.zc = zc; p.zc.marks = mk; p.zc.route = rt;
     p.order = order;
     fill_trace3_geometry( p, *conf );
     const hipStream_t s = static_cast<hipStream_t>( stream );
     hipError_t e = launch_trace3d( p, TRACE_FAST, launch_shape { 512, zc.ok ? 8 : 4, 1 }, s );
     if ( e != hipSuccess ) return fail( NUFI_ERR_DEVICE, std::string( "rho3d_noalloc: trace launch: " ) + hipGetErrorString( e ) );
     e = launch_reduce_partials( part, uint32_t( ppx ), -( conf->du * conf->dv * conf->dw ), 0, uint32_t( n_space ),
-                                uint32_t( n_space ), field_sum_group( n_space, false ), rho_dev, s );
+                                uint32_t( n_space ), field_sum_group( n_space, false ), rho_dev, s,
+                                partial_alt { zcell_window( p.zc, n, conf->Nx, conf->Ny, conf->Nz ), uint32_t( ppw ) } );
     if ( e != hipSuccess ) return fail( NUFI_ERR_DEVICE, std::string( "rho3d_noalloc: reduce launch: " ) + hipGetErrorString( e ) );
     return NUFI_OK;
 }

@@ -169,6 +169,7 @@ void trace3d_fast_kernel( trace3_params p )
 {
     extern __shared__ double lds[];
     constexpr int WPB = BLOCK / WAVE;
+    if ( p.run_if != nullptr && *p.run_if == 0 ) return;
 
     node3 id[NPT];
     double sx[NPT], sy_[NPT], sz_[NPT], vu[NPT], vv[NPT], vw[NPT];
@@ -263,7 +264,7 @@ __device__ __forceinline__ bool xm3_velocity( const trace3_params &p, const xm3_
 }
 
 // The NPT nodes a lane traces in one velocity pass of the x-major FP64 kernel.
-template <int NPT, bool MASK>
+template <int NPT, bool MASK, int G = 0>
 struct xm3_nodes
 {
     double sx[NPT], sy[NPT], sz[NPT], vu[NPT], vv[NPT], vw[NPT];
@@ -297,13 +298,13 @@ struct xm3_nodes
             }
             #pragma unroll
             for ( int r = 0; r < NPT; ++r )
-                step3_fast<MASK>( k3, C, false, false, sx[r], sy[r], sz[r], vu[r], vv[r], vw[r] );
+                step3_fast<MASK, GATHER_PF, G>( k3, C, false, false, sx[r], sy[r], sz[r], vu[r], vv[r], vw[r] );
         }
         if ( mlo == 0 )                  // slice 0: wrap3_due(0) is false
         {
             #pragma unroll
             for ( int r = 0; r < NPT; ++r )
-                step3_fast<MASK>( k3, Cb, true, false, sx[r], sy[r], sz[r], vu[r], vv[r], vw[r] );
+                step3_fast<MASK, GATHER_PF, G>( k3, Cb, true, false, sx[r], sy[r], sz[r], vu[r], vv[r], vw[r] );
         }
     }
 
@@ -324,17 +325,18 @@ struct xm3_nodes
 // 1024-thread workgroups run four waves per SIMD (128 VGPRs: the f0 evaluation
 // after each velocity pass spills, the step loop does not); 512 threads, two
 // (about 230 VGPRs, no spills; with four nodes a lane, the default shape)
-template <int BLOCK, int NPT, bool MASK>
+template <int BLOCK, int NPT, bool MASK, int G = 0>
 __global__ __launch_bounds__( BLOCK ) __attribute__(( amdgpu_waves_per_eu( BLOCK >= 1024 ? 4 : 1 ) ))
 void trace3d_xm_fast_kernel( trace3_params p )
 {
     extern __shared__ double lds[];
+    if ( p.run_if != nullptr && *p.run_if == 0 ) return;
     constexpr int WPB = BLOCK / WAVE;
     const xm3_lane a = make_xm3<WPB>( p );
     const fast3_consts k3 = make_fast3( p );
     const uint32_t st = p.st;
     csum acc { 0.0, 0.0 };
-    xm3_nodes<NPT,MASK> nd;
+    xm3_nodes<NPT,MASK,G> nd;
     const uint32_t Cn = p.chunk;
     const int64_t top = int64_t( p.n ) - 1;
     const int64_t K = ( top + int64_t( Cn ) ) / int64_t( Cn );      // chunks per pass (0 at n = 0)
@@ -784,7 +786,7 @@ hipError_t launch3_npt( const trace3_params &p, int variant, int npt, uint32_t g
     }
     // power-of-two axes: the cell index wraps by a mask, positions every 16 slices
     const bool mask = ( p.Nx & ( p.Nx - 1 ) ) == 0 && ( p.Ny & ( p.Ny - 1 ) ) == 0 && ( p.Nz & ( p.Nz - 1 ) ) == 0;
-    const bool g16 = mask && ( npt == 2 || npt == 4 ) && p.Nx == 16 && p.Ny == 16 && p.Nz == 16 && p.sy == 19 && p.sz == 19 * 19;
+    const bool g16 = mask && ( npt == 2 || npt == 4 || ( npt == 8 && variant == TRACE_FAST ) ) && p.Nx == 16 && p.Ny == 16 && p.Nz == 16 && p.sy == 19 && p.sz == 19 * 19;
     if ( variant == TRACE_FP32C )
     {
         const bool cubic = p.dx_inv == p.dy_inv && p.dx_inv == p.dz_inv;
@@ -801,7 +803,11 @@ hipError_t launch3_npt( const trace3_params &p, int variant, int npt, uint32_t g
         default: return hipErrorInvalidValue;
         }
     }
-    // eight nodes a lane are the z-cell kernel's; here four (the x-major grid and the
+    // the 16^3 grid with its strides compiled in
+    if ( g16 && npt == 8 ) return launch3( trace3d_xm_fast_kernel<BLOCK,8,true,16>, grid, BLOCK, lds, p, st );
+    if ( g16 && npt == 4 ) return launch3( trace3d_xm_fast_kernel<BLOCK,4,true,16>, grid, BLOCK, lds, p, st );
+    if ( g16 ) return launch3( trace3d_xm_fast_kernel<BLOCK,2,true,16>, grid, BLOCK, lds, p, st );
+    // eight nodes a lane exist for 16^3 only; elsewhere four (the x-major grid and the
     // partial sums do not depend on the nodes a lane holds, and 4 divides vgroup too)
     if ( npt == 8 ) npt = 4;
     switch ( npt * 2 + ( mask ? 1 : 0 ) )
@@ -871,8 +877,16 @@ hipError_t launch_trace3d( const trace3_params &p_in, int variant, const launch_
     const size_t lds = trace3d_lds_bytes( p, variant, s );
     if ( lds > 160u * 1024u ) return hipErrorInvalidValue;
 
-    // one shape of its own, whatever the caller's (legal) one
-    if ( variant == TRACE_FAST && p.mode == MODE_RHO && p.zc.ok ) return launch_trace3d_zcell( p, nullptr, st );
+    // the z-cell trace has one shape of its own; the caller's is that of the
+    // window kernel, which traces where the route says so
+    if ( variant == TRACE_FAST && p.mode == MODE_RHO && p.zc.ok )
+    {
+        const uint32_t *const window = zcell_window( p.zc, p.n, p.Nx, p.Ny, p.Nz );
+        p.zc.flag_mark = window != nullptr ? 0u : 1u;
+        const hipError_t e = launch_trace3d_zcell( p, nullptr, st );
+        if ( e != hipSuccess || window == nullptr ) return e;
+        p.run_if = window;
+    }
     if ( variant == TRACE_STRICT )
     {
         if ( p.mode == MODE_METRICS )

@@ -36,11 +36,11 @@
 // buffer and no compiled strides); metrics of 16^3 x 16^3 at n = 40 19.7 -> 5.8
 // ms (they ran the strict layout's wave tasks).  z-cells: three instead of four
 // 0.6% slower; two columns read ahead no faster; without the scheduling
-// barriers 6% slower.  Fields that mix x, y and z strongly (a product of waves
-// of amplitude 0.4 and up beside separable ones) cost more than before at 16^3:
-// the marked workgroups pay for both kernels, 48 -> 76 ms at amplitude 0.4 and
-// 61 -> 72 at 2.0 (n = 60, 24^3 velocities; 40 -> 31 at 0.1); at 20^3 150 -> 161
-// and 162 -> 163.
+// barriers 6% slower.  Fields that mix x, y and z (a product of waves
+// beside separable ones, n = 60, 24^3 velocities) are traced from z-cells while
+// that pays and from whole slices past it, decided per call (below): 16^3 mixing by
+// 0.1 of the field 38.5 -> 32.0 ms, 0.4 47.5 -> 47.3 (by marks alone 77), 2.0 60.9 ->
+// 60.7 (72); 20^3 0.1 141 -> 98, 0.2 145 -> 138 (182), 2.0 162 -> 157.
 #include "device_common.hpp"
 #include "internal.hpp"
 #include "step3d.hpp"
@@ -154,10 +154,9 @@ struct zplace
     uint32_t iw, iz, P;
     double w0, z0;
 };
-__device__ __forceinline__ zplace zc_place( const trace3_params &p )
+__device__ __forceinline__ zplace zc_place( const trace3_params &p, uint32_t b = blockIdx.x, uint32_t thread = threadIdx.x )
 {
     zplace t;
-    uint32_t b = blockIdx.x, thread = threadIdx.x;
     asm volatile( "" : "+v"( thread ) );        // formed anew where it is used: nothing of it stays in registers
     const uint32_t gb = b % p.zc.ngb; b /= p.zc.ngb;
     const uint32_t tile = b % p.zc.tiles; b /= p.zc.tiles;
@@ -233,6 +232,11 @@ void trace3d_zcell_kernel( trace3_params p )
 {
     extern __shared__ __align__( 16 ) char zlds[];
     constexpr int NPT = 8;                                            // nodes a lane
+    if ( p.zc.route != nullptr && p.zc.route->window != 0 )
+    {
+        if ( threadIdx.x == 0 ) p.zc.marks[ blockIdx.x ] = p.zc.flag_mark;
+        return;
+    }
     const uint32_t tid = threadIdx.x, lane = tid % WAVE, threads = blockDim.x;
     const uint32_t wave = __builtin_amdgcn_readfirstlane( tid / WAVE ), waves = threads / WAVE;
     const uint32_t nzc = p.zc.nzc, plane = G > 0 ? uint32_t( ( G + 3 ) * ( G + 3 ) ) : p.sz;
@@ -588,6 +592,154 @@ void trace3d_zslice_kernel( trace3_params p )
     zc_write<MODE,NM>( p, zc_place( p ), acc );
 }
 
+// ---- which kernel traces a call -----------------------------------------------
+// The z-cell kernel pays where the nodes of a workgroup keep together in z.  A
+// field that mixes the axes strongly drives them apart, and then the marked
+// workgroups pay for both kernels: up to twice the time of whole slices alone.
+// Two launches ahead of the trace decide from the slices it will read, so that
+// the result depends on the history alone and not on earlier calls or on how a
+// caller cuts the nodes (6 us together where the first settles it):
+//
+// trace3d_spread_kernel bounds how far apart two nodes of a workgroup can get
+// while their z is about the same: a slice's z kick differs over (x, y) by at
+// most the spread of its coefficients' z differences (the spline's slope is a
+// convex combination of them), and slice m's kick is followed by m drifts.  Up to
+// ZC_SPREAD_SURE cells (a sum of one wave per axis: 0) no node leaves its window.
+// The bound knows nothing of phases and of the nodes' own motion, and is 3 to 5 times
+// what they do.  With at most ZC_FEW workgroups, where more launches would show,
+// it decides alone, at ZC_SPREAD_FEW (8^3 x 12^3 at n = 40, z-cells / whole slices:
+// bound 4.2 0.76 / 1.07 ms, 4.6 0.75 / 1.07, 7.0 1.47 / 1.09, 7.7 1.40 / 1.09).
+//
+// trace3d_scout_kernel runs where the bound left it open: the
+// nodes of one velocity pass of up to ZC_SCOUTS workgroups, a node a lane, from
+// whole slices in LDS, counting the wave-steps with a lane outside the window of
+// the workgroup's first node.  They step over every second or fourth slice of a
+// long history: one node a lane makes the step a bare chain of latencies (3 us).
+//
+// What a workgroup's misses cost: ZC_MISS_COST times the share of its steps in
+// which one of its waves missed (a missed node-step is 13 times as dear, and the
+// others wait for it at the barrier), at most ZC_COST_CAP, in units of its trace.
+// On average whole slices are worth taking from, in 1/64: 7 at 16^3, where the
+// window kernel has its strides compiled in (mixing by 0.15 of the field: cost 0.04,
+// 32 ms against its 40; 0.09: 34 / 40; 0.13: 45 / 42), and for windows of two z-cells
+// (24 x 20 x 12: 0.01 22 / 26, 0.44 35 / 26); 19 elsewhere (20^3: 0.12 117 / 136,
+// 0.27 121 / 136, 0.40 174 / 136; 20 x 18 x 20: 0.23 26 / 30, 0.31 33 / 30).
+constexpr unsigned long long ZC_FIX = 65536;                          // sums in 1/65536
+constexpr double ZC_SPREAD_SURE = 1.0, ZC_SPREAD_FEW = 5.5;
+constexpr uint32_t ZC_SCOUTS = 256, ZC_FEW = 2 * ZC_SCOUTS;
+constexpr unsigned long long ZC_MISS_COST = 13, ZC_COST_CAP = 24;     // the cap in 1/16
+constexpr unsigned long long ZC_WORTH = 19, ZC_WORTH_CLOSE = 7;
+__host__ __device__ inline uint32_t zc_all( const trace3_params &p ) { return p.Nz * p.Nw * p.zc.tiles * p.zc.ngb; }   // workgroups of the grid
+__host__ __device__ inline uint32_t scout_stride( uint64_t n ) { return n >= 32 ? 4u : n >= 16 ? 2u : 1u; }
+
+__global__ __launch_bounds__( 1024 )
+void trace3d_spread_kernel( trace3_params p )
+{
+    __shared__ double most_w[16];
+    const uint32_t m = blockIdx.x, lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, P = p.Nx * p.Ny;
+    const double *const c = p.hist + size_t( m ) * p.st;
+    double most = 0.0;
+    bool odd = false;                                                 // not finite: no bound
+    for ( uint32_t k = wave; k < p.Nz; k += 16 )
+    {
+        double lo = __builtin_inf(), hi = -__builtin_inf();
+        #pragma unroll 4
+        for ( uint32_t e = lane; e < P; e += WAVE )
+        {
+            const uint32_t y = e / p.Nx, at = k * p.sz + y * p.sy + ( e - y * p.Nx );
+            const double d = c[ at + p.sz ] - c[at];
+            odd = odd || !( d - d == 0.0 );
+            lo = fmin( lo, d ); hi = fmax( hi, d );
+        }
+        #pragma unroll
+        for ( int off = 32; off > 0; off >>= 1 )
+        {
+            lo = fmin( lo, __shfl_xor( lo, off ) ); hi = fmax( hi, __shfl_xor( hi, off ) );
+        }
+        most = fmax( most, hi - lo );
+    }
+    if ( __builtin_amdgcn_ballot_w64( odd ) != 0 ) most = __builtin_inf();
+    if ( lane == 0 ) most_w[wave] = most;
+    __syncthreads();
+    if ( threadIdx.x != 0 ) return;
+    for ( int w = 1; w < 16; ++w ) most = fmax( most, most_w[w] );
+    constexpr double CAP = 16777216.0;
+    const double cells = most * p.zc.k.cd[2] * p.zc.k.cd[2] * double( m );
+    zcell_route *const r = p.zc.route;
+    atomicAdd( &r->spread, (unsigned long long)( ( cells < CAP ? cells : CAP ) * double( ZC_FIX ) ) );
+    __threadfence();
+    if ( atomicAdd( &r->arrived[0], 1u ) != gridDim.x - 1 ) return;
+    const unsigned long long all = atomicExch( &r->spread, 0ull );
+    r->arrived[0] = 0;
+    r->last_spread = all; r->last_cost = 0;
+    const bool few = zc_all( p ) <= ZC_FEW;
+    r->window = few && double( all ) > ZC_SPREAD_FEW * double( ZC_FIX ) ? 1u : 0u;
+    r->scout = !few && double( all ) > ZC_SPREAD_SURE * double( ZC_FIX ) ? 1u : 0u;
+}
+
+template <bool MASK, int G>
+__global__ __launch_bounds__( 512 ) __attribute__(( amdgpu_waves_per_eu( 2, 2 ) ))
+void trace3d_scout_kernel( trace3_params p )
+{
+    extern __shared__ __align__( 16 ) double zfull[];
+    if ( p.zc.route->scout == 0 ) return;                             // uniform
+    const uint32_t tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE, waves = blockDim.x / WAVE, st = p.st;
+    // scattered over the workgroups by golden-ratio steps, and over their passes
+    const uint32_t all = zc_all( p );
+    const uint32_t b = uint32_t( ( uint64_t( blockIdx.x * 2654435769u ) * all ) >> 32 );
+    const uint32_t pass = ( blockIdx.x * 5u ) % ( ( p.zc.vg + 7 ) / 8 );
+    // lane 0 of each wave is the workgroup's first node, whose window it is
+    const zplace t = zc_place( p, b, lane == 0 ? 0u : tid );
+    double x = double( t.a.ix ), y = double( t.a.iy ), z = t.z0, u, v, w = t.w0;
+    (void)zc_velocity( p, t.a, t.iw, pass * 8 + ( lane == 0 ? 0u : ( 3 * wave ) % 8 ), u, v );
+    fast3_consts k3 = make_fast3( p );
+    const int n = int( p.n ), Nzi = int( p.Nz ), stride = int( scout_stride( p.n ) );
+    const double ds = double( stride );
+    k3.cdx *= ds; k3.cdy *= ds; k3.cdz *= ds; k3.kx *= ds; k3.ky *= ds; k3.kz *= ds;
+    const double zoff = 0.5 * ( double( p.zc.nzc ) - 1.0 );
+    auto buffer = [&]( int i ) __attribute__(( always_inline )) { return zfull + ( ( i & 1 ) && p.dma ? st + 2u : 0u ); };
+    auto copy = [&]( int i, int m ) __attribute__(( always_inline ))
+    {
+        const double *src = p.hist + size_t( m ) * st;
+        const uint32_t mis = uint32_t( reinterpret_cast<uintptr_t>( src ) & 15u ) / 8u;
+        dma_copy16( buffer( i ), src - mis, ( st + mis + 1 ) / 2, waves );
+    };
+    uint32_t missed = 0;
+    if ( p.dma ) { copy( 0, n - 1 ); dma_publish(); }
+    for ( int i = 0, m = n - 1; m >= 0; ++i, m -= stride )
+    {
+        if ( p.dma ) { if ( m >= stride ) copy( i + 1, m - stride ); }
+        else { __syncthreads(); copy( 0, m ); dma_publish(); }
+        const double *C = buffer( i ) + ( reinterpret_cast<uintptr_t>( p.hist + size_t( m ) * st ) & 15u ) / 8u;
+        if ( MASK ) { rewrap3( x, k3.Nxd, k3.iNx ); rewrap3( y, k3.Nyd, k3.iNy ); rewrap3( z, k3.Nzd, k3.iNz ); }
+        step3_fast<MASK,GATHER_PF,G>( k3, C, false, false, x, y, z, u, v, w );
+        double z0 = __shfl( z, 0 ) - zoff;
+        z0 = fma( -k3.Nzd, floor( z0 * k3.iNz ), z0 );
+        const uint32_t rel = zc_rel<MASK>( int( floor( z ) ), int( zc_held( int( z0 ), uint32_t( Nzi ) ) ), Nzi );
+        missed += __builtin_amdgcn_ballot_w64( rel >= p.zc.nzc ) != 0 ? 1u : 0u;
+        if ( p.dma ) dma_publish();
+    }
+    __syncthreads();                                                  // the slices are read
+    uint32_t *const per_wave = reinterpret_cast<uint32_t*>( zfull );
+    if ( lane == 0 ) per_wave[wave] = missed;
+    __syncthreads();
+    if ( tid != 0 ) return;
+    unsigned long long out = 0;
+    for ( uint32_t q = 0; q < waves; ++q ) out += per_wave[q];
+    const unsigned long long steps = ( p.n + stride - 1 ) / stride, cap = ZC_COST_CAP * ZC_FIX / 16;
+    unsigned long long cost = ZC_MISS_COST * ZC_FIX * out / steps;
+    if ( cost > cap ) cost = cap;
+    zcell_route *const r = p.zc.route;
+    atomicAdd( &r->cost, cost );
+    __threadfence();
+    if ( atomicAdd( &r->arrived[1], 1u ) != gridDim.x - 1 ) return;
+    const unsigned long long mean = atomicExch( &r->cost, 0ull ) / gridDim.x;
+    r->arrived[1] = 0;
+    r->last_cost = mean;
+    const unsigned long long worth = G == 16 || p.zc.nzc < 3 ? ZC_WORTH_CLOSE : ZC_WORTH;
+    r->window = mean > worth * ZC_FIX / 64 ? 1u : 0u;
+}
+
 template <int MODE>
 const void *zslice_kernel( bool mask, bool g16 )
 {
@@ -686,21 +838,36 @@ hipError_t launch_trace3d_zcell( const trace3_params &p_in, uint32_t *tasks, hip
     const bool metrics = p.mode == MODE_METRICS;
     if ( p.zc.marks == nullptr ) return hipErrorInvalidValue;
     const void *k = nullptr;
-    k = metrics ? zcell_kernel<MODE_METRICS>( mask, g16 ) : zcell_kernel<MODE_RHO>( mask, g16 );
-    const size_t lds = zcell_lds( p.zc.nzc, p.Nx * ( p.Ny + 3 ), p.zc.szp );
-    hipError_t e = hipFuncSetAttribute( k, hipFuncAttributeMaxDynamicSharedMemorySize, int( lds ) );
-    if ( e != hipSuccess ) return e;
     void *args[] = { &p };
-    e = hipLaunchKernel( k, dim3( uint32_t( grid ) ), dim3( threads ), args, lds, st );
-    if ( e != hipSuccess ) return e;
-    if ( tasks ) *tasks = uint32_t( grid ) * ( threads / WAVE );
-    if ( p.n == 0 || p.zc.nzc >= p.Nz ) return hipGetLastError();      // no window to leave
+    hipError_t e;
     p.dma = fast3_dma( 1, p.st ) ? 1u : 0u;
     // 16-byte words of a slice, whichever half of one it starts in
     const size_t full = p.dma ? 2 * size_t( p.st + 2 ) * sizeof(double) : size_t( ( p.st + 1 ) / 2 ) * 16u;
+    auto launch = [&]( const void *f, uint32_t blocks, uint32_t block, size_t lds )
+    {
+        hipError_t err = lds > 0 ? hipFuncSetAttribute( f, hipFuncAttributeMaxDynamicSharedMemorySize, int( lds ) ) : hipSuccess;
+        if ( err == hipSuccess ) err = hipLaunchKernel( f, dim3( blocks ), dim3( block ), args, lds, st );
+        return err;
+    };
+    if ( zcell_routed( p.zc, p.n, p.Nz ) )
+    {
+        const uint32_t z_first = p.zc.z_first;
+        p.zc.z_first = 0;                                  // of the whole grid, whatever slab the call traces
+        e = launch( reinterpret_cast<const void*>( trace3d_spread_kernel ), uint32_t( p.n ), 1024, 0 );
+        if ( e != hipSuccess ) return e;
+        k = g16 ? reinterpret_cast<const void*>( trace3d_scout_kernel<true,16> )
+                : mask ? reinterpret_cast<const void*>( trace3d_scout_kernel<true,0> ) : reinterpret_cast<const void*>( trace3d_scout_kernel<false,0> );
+        if ( zc_all( p ) > ZC_FEW && ( e = launch( k, ZC_SCOUTS, threads, full ) ) != hipSuccess ) return e;
+        p.zc.z_first = z_first;
+    }
+    else p.zc.route = nullptr;
+    k = metrics ? zcell_kernel<MODE_METRICS>( mask, g16 ) : zcell_kernel<MODE_RHO>( mask, g16 );
+    const size_t lds = zcell_lds( p.zc.nzc, p.Nx * ( p.Ny + 3 ), p.zc.szp );
+    if ( ( e = launch( k, uint32_t( grid ), threads, lds ) ) != hipSuccess ) return e;
+    if ( tasks ) *tasks = uint32_t( grid ) * ( threads / WAVE );
+    if ( p.n == 0 || p.zc.nzc >= p.Nz ) return hipGetLastError();      // no window to leave
     k = metrics ? zslice_kernel<MODE_METRICS>( mask, g16 ) : zslice_kernel<MODE_RHO>( mask, g16 );
-    if ( ( e = hipFuncSetAttribute( k, hipFuncAttributeMaxDynamicSharedMemorySize, int( full ) ) ) != hipSuccess ) return e;
-    if ( ( e = hipLaunchKernel( k, dim3( uint32_t( grid ) ), dim3( threads ), args, full, st ) ) != hipSuccess ) return e;
+    if ( ( e = launch( k, uint32_t( grid ), threads, full ) ) != hipSuccess ) return e;
     return hipGetLastError();
 }
 

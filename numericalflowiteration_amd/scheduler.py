@@ -245,6 +245,15 @@ class GpuScheduler:
         self._check(self._lib.nufi_trace_timing(self._ctx, ctypes.byref(n), _ptr(ms), _ptr(cs)))
         return int(n.value), float(ms[0]), float(cs[0])
 
+    def trace3d_route(self) -> dict:
+        """How the last 3D FP64 trace ran (nufi_trace3d_route): whether the z-cell
+        kernel takes the grid, whether the history had it trace from whole slices
+        instead, the bound in cells, the cost of misses, workgroups redone and in all."""
+        out = (ctypes.c_uint64 * 6)()
+        self._check(self._lib.nufi_trace3d_route(self._ctx, out))
+        return dict(zcell=bool(out[0]), window=bool(out[1]), spread=out[2] / 65536.0, cost=out[3] / 65536.0,
+                    marked=int(out[4]), workgroups=int(out[5]))
+
 
 
 
