@@ -706,14 +706,14 @@ int nufi_compute_metrics( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_
             p.sy = c->sy; p.sz = c->sz; p.st = c->st; p.wpx = c->m_wpx;
             p.l_first = uint32_t( l0 ); p.n_tasks = uint32_t( tasks ); p.order = uint32_t( c->order );
             fill_trace3_geometry( p, g );
-            if ( variant == TRACE_FAST && c->zc.ok )
+            if ( variant == TRACE_FAST && zcell_metrics( c->zc, c->m_nodes, c->st ) )
             {
                 uint32_t waves = 0;
                 p.n_count = uint32_t( l1 - l0 + 1 ); p.zc = c->zc;
                 // where the route leaves the z-cells: small slices, cheap to stage, in wave
                 // tasks (11 x 13 x 9, mixing by 2: 1.9 ms, by trace3d_zslice_kernel 2.5),
                 // others by that (16^3 116 / 73 ms)
-                const bool wave_tasks = zcell_routed( c->zc, n, g.Nz ) && c->st <= 5120;
+                const bool wave_tasks = zcell_routed( c->zc, n, g.Nz ) && c->st <= WAVE_TASK_SLICE;
                 p.zc.flag_mark = wave_tasks ? 0u : 1u;
                 e = launch_trace3d_zcell( p, &waves, c->stream );
                 if ( e == hipSuccess && wave_tasks )

@@ -270,6 +270,17 @@ inline bool zcell_routed( const zcell_plan &z, uint64_t n, uint64_t Nz )
 {
     return z.ok && z.route != nullptr && z.nzc < Nz && n >= ZCELL_ROUTE_MIN;
 }
+// Whether the metrics of a grid are traced from z-cells (or whole slices in their
+// place) and not in wave tasks.  With less than a round of workgroups on the chip
+// a z-cell trace takes a round's time all the same (20 us a slice), wave tasks 15 to 21 ps
+// a node and slice while the slice they stage is small: n = 40, 4^3 x 8^3 289 / 80 us,
+// 6^3 x 8^3 410 / 105, 8^3 x 9^3 396 / 278, 8^3 x 12^3 777 / 571, 9x10x11 x 9x10x9 849 / 609;
+// above, 10^3 x 12^3 886 / 1184, 8^3 x 16^3 795 / 1090, 13x14x15 x 10^3 1392 / 2399.
+constexpr uint32_t WAVE_TASK_SLICE = 5120;      // reals
+inline bool zcell_metrics( const zcell_plan &z, uint64_t nodes, uint32_t st )
+{
+    return z.ok && !( nodes < ( 1u << 20 ) && st <= WAVE_TASK_SLICE );
+}
 // The flag by which the window kernel traces rho in the z-cell workgroups' place,
 // null where it never does.  At 16^3 its compiled strides and eight nodes a lane
 // beat trace3d_zslice_kernel (n = 60, 24^3 velocities, mixing by 0.4: 47 against 55 ms);

@@ -141,3 +141,21 @@ def test_replayed_graph(N, V):
             e, h = steps(s, mix, True)
             assert np.array_equal(e, want[mix][0]) and np.array_equal(h, want[mix][1])
             rho_of(s, 3)
+
+
+@pytest.mark.parametrize("N,V", [((8, 8, 8), (16, 8, 15)), ((8, 8, 8), (16, 8, 16)), ((9, 7, 10), (13, 8, 17)), ((10, 9, 8), (13, 8, 14))])
+def test_metrics_on_both_sides_of_the_wave_tasks(N, V):
+    """Metrics go to wave tasks below 2^20 nodes of small slices, to z-cells above."""
+    c = make(N, V)
+    hist = history(c, 18, 0.1)
+    with nufi.GpuScheduler(c) as s:
+        s.upload_history(hist, 0, 18)
+        for n in (1, 17):
+            check_metrics(c, n, hist, s)
+        got, parts = np.zeros(4), np.zeros(4)
+        s.compute_metrics(17)
+        s.download_metrics(got)
+        for a, b in ((0, 1000), (1000, c.n_nodes())):
+            s.compute_metrics(17, a, b)
+            s.download_metrics(parts)
+        assert np.max(np.abs(parts - got) / np.abs(got)) <= 1e-13
