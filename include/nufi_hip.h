@@ -147,7 +147,9 @@ int nufi_synchronize(nufi_ctx *ctx);
 int nufi_compute_rho(nufi_ctx *ctx, uint64_t n, uint64_t q_begin, uint64_t q_end);
 /* Synchronises and ADDS the device rho (Nx*Ny*Nz reals) into rho_accum. */
 int nufi_download_rho(nufi_ctx *ctx, double *rho_accum);
-/* Copies slice n from history_base + n*stride_t (host) to the device. */
+/* Copies slice n from history_base + n*stride_t (host) to the device.  3D traces
+ * read its pads as they stand; slices whose pads are not the periodic copies of
+ * their interior (every slice the library writes has those) take slower kernels. */
 int nufi_upload_phi(nufi_ctx *ctx, uint64_t n, const double *history_base);
 /*
  * Metrics [int f, int f^2, kinetic energy, entropy] of nodes [q_begin,q_end)

@@ -42,6 +42,8 @@ struct nufi_ctx
     uint32_t ppx = 0;          // x-major partials per spatial point (fast; 1D FP32C); 3D: the window kernel's
     uint32_t vgroup = 0;       // 3D x-major: velocities per partial
     zcell_plan zc {};          // 3D fast FP64 (rho and metrics): the z-cell kernel's layout, zc.ok where it runs
+    std::vector<uint8_t> odd_pads;   // zc.ok: per slice, 1 where an uploaded one's pads are no periodic copies
+    uint64_t n_odd = 0;              // and how many those are
     int field_ok = 0;          // 1: one-workgroup field solve; 2: the multi-workgroup one; 0: none
     double2 *lw0 = nullptr, *lw1 = nullptr;   // multi-workgroup solve: two complex buffers
     double *lpart = nullptr;                  // and its energy partials
@@ -199,17 +201,49 @@ int build_tables( nufi_ctx *c )
     return NUFI_OK;
 }
 
-// partials per spatial point of the rho kernel in use
-uint32_t rho_ppx( const nufi_ctx *c )
+// Whether slices below n may be traced from z-cells, which are formed as if a
+// slice went on periodically: other pads are read by the window and wave-task
+// kernels only.
+bool zcell_slices( const nufi_ctx *c, uint64_t n )
+{
+    if ( !c->zc.ok ) return false;
+    for ( uint64_t m = 0; c->n_odd > 0 && m < n; ++m ) if ( c->odd_pads[m] ) return false;
+    return true;
+}
+
+// Whether the pads of a 3D slice (host) are the periodic copies.
+bool periodic_pads( const nufi_config &g, const double *s )
+{
+    const uint64_t ex = g.Nx + 3, ey = g.Ny + 3, ez = g.Nz + 3;
+    for ( uint64_t k = 0; k < ez; ++k )
+        for ( uint64_t j = 0; j < ey; ++j )
+        {
+            const double *row = s + ( k * ey + j ) * ex, *base = s + ( ( k % g.Nz ) * ey + j % g.Ny ) * ex;
+            if ( row != base && std::memcmp( row, base, ex * sizeof(double) ) != 0 ) return false;
+            for ( uint64_t i = g.Nx; row == base && i < ex; ++i )
+                if ( std::memcmp( row + i, row + i % g.Nx, sizeof(double) ) != 0 ) return false;
+        }
+    return true;
+}
+
+void set_odd_pads( nufi_ctx *c, uint64_t n, bool odd )
+{
+    if ( !c->zc.ok || ( c->odd_pads[n] != 0 ) == odd ) return;
+    c->odd_pads[n] = odd ? 1 : 0;
+    c->n_odd += odd ? 1 : uint64_t( -1 );
+}
+
+// partials per spatial point of the rho kernel in use at step n
+uint32_t rho_ppx( const nufi_ctx *c, uint64_t n )
 {
     const bool xm = c->variant == TRACE_FAST || ( c->dim == 1 && c->variant == TRACE_FP32C );
-    return xm ? ( c->zc.ok ? c->zc.ppx : c->ppx ) : c->wpx;
+    return xm ? ( zcell_slices( c, n ) ? c->zc.ppx : c->ppx ) : c->wpx;
 }
 
 // and those of the window kernel where step n may take it
 partial_alt rho_alt( const nufi_ctx *c, uint64_t n )
 {
-    if ( c->dim != 3 || c->variant != TRACE_FAST ) return partial_alt {};
+    if ( c->dim != 3 || c->variant != TRACE_FAST || !zcell_slices( c, n ) ) return partial_alt {};
     return partial_alt { zcell_window( c->zc, n, c->conf.Nx, c->conf.Ny, c->conf.Nz ), c->ppx };
 }
 
@@ -339,7 +373,8 @@ int launch_trace( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_end, uin
         p.Nu = uint32_t( c->conf.Nu ); p.Nv = uint32_t( c->conf.Nv ); p.Nw = uint32_t( c->conf.Nw );
         p.sy = c->sy; p.sz = c->sz; p.st = c->st; p.st32 = c->st32; p.wpx = c->wpx;
         p.l_first = uint32_t( l0 ); p.n_tasks = uint32_t( tasks );
-        p.n_count = uint32_t( l1 - l0 + 1 ); p.vgroup = c->vgroup; p.ppx = c->ppx; p.zc = c->zc;
+        p.n_count = uint32_t( l1 - l0 + 1 ); p.vgroup = c->vgroup; p.ppx = c->ppx;
+        if ( zcell_slices( c, n ) ) p.zc = c->zc;
         p.order = uint32_t( c->order );
         fill_trace3_geometry( p, c->conf );
         e = launch_trace3d( p, c->variant, c->shape, c->stream );
@@ -378,7 +413,6 @@ field_params base_field( nufi_ctx *c )
     const bool fp32c = c->precision == NUFI_FP32C;
     f.rx = make_radices( f.Nx, fp32c ); f.ry = make_radices( f.Ny, fp32c ); f.rz = make_radices( f.Nz, fp32c );
     f.sum_group = field_sum_group( f.N, fp32c );
-    f.wpx = rho_ppx( c );
     f.weight = rho_weight( c );
     f.tw_x = c->tw_x; f.tw_y = c->tw_y; f.tw_z = c->tw_z;
     f.ewt = c->ewt;
@@ -561,6 +595,7 @@ int nufi_create( const nufi_config *conf, const nufi_config *conf_metrics, int o
     if ( ( rc = dev_alloc( c, &c->mpartials, 4 * m_waves, "metric partials" ) ) ) return bail( rc );
     if ( c->field_ok && ( rc = build_tables( c ) ) ) return bail( rc );
     c->host_rho.assign( c->n_space, 0.0 );
+    if ( c->zc.ok ) c->odd_pads.assign( slices, 0 );
     default_shape( c );
     *out = c;
     return NUFI_OK;
@@ -607,14 +642,14 @@ int nufi_compute_rho( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_end 
     if ( q_begin == q_end )
     {
         // empty range: the device rho becomes zero, so download_rho adds nothing
-        hipError_t e = launch_reduce_partials( c->partials, rho_ppx( c ), 0.0, 0, 0, uint32_t( c->n_space ), 1, c->rho, c->stream );
+        hipError_t e = launch_reduce_partials( c->partials, rho_ppx( c, n ), 0.0, 0, 0, uint32_t( c->n_space ), 1, c->rho, c->stream );
         if ( e != hipSuccess ) return hip_fail( c, e, "reduce launch" );
         return NUFI_OK;
     }
     uint64_t first, count;
     int rc = launch_trace( c, n, q_begin, q_end, &first, &count );
     if ( rc ) return rc;
-    hipError_t e = launch_reduce_partials( c->partials, rho_ppx( c ), rho_weight( c ), uint32_t( first ), uint32_t( count ),
+    hipError_t e = launch_reduce_partials( c->partials, rho_ppx( c, n ), rho_weight( c ), uint32_t( first ), uint32_t( count ),
                                            uint32_t( c->n_space ), field_sum_group( c->n_space, c->precision == NUFI_FP32C ),
                                            c->rho, c->stream, rho_alt( c, n ) );
     if ( e != hipSuccess ) return hip_fail( c, e, "reduce launch" );
@@ -639,6 +674,7 @@ int nufi_upload_phi( nufi_ctx *c, uint64_t n, const double *history_base )
     if ( n > c->conf.Nt ) return fail( c, NUFI_ERR_RANGE, "upload_phi: time step out of range" );
     HIP_TRY( c, hipSetDevice( c->device ) );
     double *dst = c->hist + n * c->st;
+    if ( c->zc.ok ) set_odd_pads( c, n, !periodic_pads( c->conf, history_base + n * c->st ) );
     HIP_TRY( c, hipMemcpyAsync( dst, history_base + n * c->st, c->st * sizeof(double), hipMemcpyHostToDevice, c->stream ) );
     hipError_t e = launch_slice_tables( c->dim, dst, c->st, uint32_t( c->conf.Nx ),
                                         c->dhist ? c->dhist + n * c->sd : nullptr,
@@ -706,7 +742,7 @@ int nufi_compute_metrics( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_
             p.sy = c->sy; p.sz = c->sz; p.st = c->st; p.wpx = c->m_wpx;
             p.l_first = uint32_t( l0 ); p.n_tasks = uint32_t( tasks ); p.order = uint32_t( c->order );
             fill_trace3_geometry( p, g );
-            if ( variant == TRACE_FAST && zcell_metrics( c->zc, c->m_nodes, c->st ) )
+            if ( variant == TRACE_FAST && zcell_metrics( c->zc, c->m_nodes, c->st ) && zcell_slices( c, n + 1 ) )
             {
                 uint32_t waves = 0;
                 p.n_count = uint32_t( l1 - l0 + 1 ); p.zc = c->zc;
@@ -764,7 +800,9 @@ static int step_async( nufi_ctx *c, uint64_t n, double *rho_out )
     field_params f = base_field( c );
     f.mode = FIELD_STEP;
     f.partials = c->partials;
+    f.wpx = rho_ppx( c, n );
     f.alt = rho_alt( c, n );
+    set_odd_pads( c, n, false );             // the slice this step writes is periodic
     if ( uint64_t( f.alt.sel ? std::max( f.wpx, f.alt.count ) : f.wpx ) * c->n_space > ( uint64_t( 1 ) << 16 ) )
     {
         // many partials (3D): one thread per point over many workgroups sums them
@@ -812,7 +850,7 @@ int nufi_run( nufi_ctx *c, uint64_t n_begin, uint64_t n_end, double *energies )
     if ( n_end > n_begin && !c->field_ok )
         return fail( c, NUFI_ERR_UNSUPPORTED, "step: grid too large for the single-workgroup field solve" );
     HIP_TRY( c, hipSetDevice( c->device ) );
-    if ( c->use_graph && !c->timing && n_end > n_begin )
+    if ( c->use_graph && !c->timing && n_end > n_begin && c->n_odd == 0 )     // a graph keeps the kernels of its capture
     {
         // the trace and field launches of every step, captured once and replayed
         // (no memset or event in the captured range: every buffer a step reads

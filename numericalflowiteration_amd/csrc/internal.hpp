@@ -113,6 +113,7 @@ struct zcell_route
     uint32_t window;         // 1: whole slices (trace3d_zslice_kernel or the window kernel), not z-cells
     uint32_t scout;          // 1: the bound left it open, scouts decide
     uint32_t arrived[2];     // workgroups of the two deciding kernels that are done
+    uint32_t odd_pads;       // slices whose pads are no periodic copies
     unsigned long long spread, cost;           // their sums (integers: any order gives the same)
     unsigned long long last_spread, last_cost; // of the last call, for reports
 };
@@ -128,6 +129,7 @@ struct zcell_plan
     uint32_t *marks;         // per workgroup: 1 where the window did not hold its nodes
     uint32_t flag_mark;      // per launch: the mark of a workgroup that the route takes off the z-cell kernel
     zcell_route *route;
+    uint32_t check_pads;     // the history comes unchecked: slices whose pads are no periodic copies go to whole slices
     zcell_consts k;
 };
 inline size_t zcell_lds( uint32_t nzc, uint32_t cols, uint32_t szp )
@@ -266,9 +268,13 @@ hipError_t launch_trace3d_zcell( const trace3_params &p, uint32_t *tasks, hipStr
 // of twice the thermal energy at 16^3), and the deciding launches (6 us) are up to a
 // tenth of a call.
 constexpr uint64_t ZCELL_ROUTE_MIN = 16;
+__host__ __device__ inline bool zcell_decides( const zcell_plan &z, uint64_t n, uint64_t Nz )
+{
+    return z.nzc < Nz && n >= ZCELL_ROUTE_MIN;
+}
 inline bool zcell_routed( const zcell_plan &z, uint64_t n, uint64_t Nz )
 {
-    return z.ok && z.route != nullptr && z.nzc < Nz && n >= ZCELL_ROUTE_MIN;
+    return z.ok && z.route != nullptr && ( z.check_pads ? n > 0 : zcell_decides( z, n, Nz ) );
 }
 // Whether the metrics of a grid are traced from z-cells (or whole slices in their
 // place) and not in wave tasks.  With less than a round of workgroups on the chip

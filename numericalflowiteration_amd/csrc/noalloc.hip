@@ -122,7 +122,7 @@ extern "C" int nufi_rho3d_noalloc( const nufi_config *conf, uint64_t n, const do
     p.sy = uint32_t( sy ); p.sz = uint32_t( sz ); p.st = uint32_t( st ); p.st32 = uint32_t( ( st + 3 ) & ~uint64_t( 3 ) );
     p.wpx = uint32_t( wpx );
     p.l_first = 0; p.n_tasks = uint32_t( n_space * wpx ); p.n_count = uint32_t( n_space );
-    p.vgroup = vgroup; p.ppx = uint32_t( ppw ); p.zc = zc; p.zc.marks = mk; p.zc.route = rt;
+    p.vgroup = vgroup; p.ppx = uint32_t( ppw ); p.zc = zc; p.zc.marks = mk; p.zc.route = rt; p.zc.check_pads = 1;
     p.order = order;
     fill_trace3_geometry( p, *conf );
     const hipStream_t s = static_cast<hipStream_t>( stream );

@@ -610,6 +610,10 @@ void trace3d_zslice_kernel( trace3_params p )
 // it decides alone, at ZC_SPREAD_FEW (8^3 x 12^3 at n = 40, z-cells / whole slices:
 // bound 4.2 0.76 / 1.07 ms, 4.6 0.75 / 1.07, 7.0 1.47 / 1.09, 7.7 1.40 / 1.09).
 //
+// It also looks at the pads of a history that nobody has looked at yet
+// (nufi_rho3d_noalloc): z-cells are formed as if the slice went on periodically,
+// whole slices are read with their pads.
+//
 // trace3d_scout_kernel runs where the bound left it open: the
 // nodes of one velocity pass of up to ZC_SCOUTS workgroups, a node a lane, from
 // whole slices in LDS, counting the wave-steps with a lane outside the window of
@@ -659,6 +663,18 @@ void trace3d_spread_kernel( trace3_params p )
         most = fmax( most, hi - lo );
     }
     if ( __builtin_amdgcn_ballot_w64( odd ) != 0 ) most = __builtin_inf();
+    bool pads = false;
+    if ( p.zc.check_pads )                                            // uniform
+    {
+        const uint32_t sy = p.sy, rows = p.Ny + 3;
+        for ( uint32_t e = threadIdx.x; e < p.st; e += 1024 )
+        {
+            const uint32_t row = e / sy, i = e - row * sy, k = row / rows, j = row - k * rows;
+            const uint32_t from = ( k % p.Nz ) * p.sz + ( j % p.Ny ) * sy + i % p.Nx;
+            pads = pads || ( from != e && __double_as_longlong( c[e] ) != __double_as_longlong( c[from] ) );
+        }
+    }
+    pads = __syncthreads_or( pads ? 1 : 0 ) != 0;
     if ( lane == 0 ) most_w[wave] = most;
     __syncthreads();
     if ( threadIdx.x != 0 ) return;
@@ -667,14 +683,16 @@ void trace3d_spread_kernel( trace3_params p )
     const double cells = most * p.zc.k.cd[2] * p.zc.k.cd[2] * double( m );
     zcell_route *const r = p.zc.route;
     atomicAdd( &r->spread, (unsigned long long)( ( cells < CAP ? cells : CAP ) * double( ZC_FIX ) ) );
+    if ( pads ) atomicAdd( &r->odd_pads, 1u );
     __threadfence();
     if ( atomicAdd( &r->arrived[0], 1u ) != gridDim.x - 1 ) return;
     const unsigned long long all = atomicExch( &r->spread, 0ull );
+    const uint32_t odd_slices = atomicExch( &r->odd_pads, 0u );
     r->arrived[0] = 0;
     r->last_spread = all; r->last_cost = 0;
-    const bool few = zc_all( p ) <= ZC_FEW;
-    r->window = few && double( all ) > ZC_SPREAD_FEW * double( ZC_FIX ) ? 1u : 0u;
-    r->scout = !few && double( all ) > ZC_SPREAD_SURE * double( ZC_FIX ) ? 1u : 0u;
+    const bool few = zc_all( p ) <= ZC_FEW, open = odd_slices == 0 && zcell_decides( p.zc, p.n, p.Nz );
+    r->window = odd_slices != 0 || ( open && few && double( all ) > ZC_SPREAD_FEW * double( ZC_FIX ) ) ? 1u : 0u;
+    r->scout = open && !few && double( all ) > ZC_SPREAD_SURE * double( ZC_FIX ) ? 1u : 0u;
 }
 
 template <bool MASK, int G>
@@ -857,7 +875,7 @@ hipError_t launch_trace3d_zcell( const trace3_params &p_in, uint32_t *tasks, hip
         if ( e != hipSuccess ) return e;
         k = g16 ? reinterpret_cast<const void*>( trace3d_scout_kernel<true,16> )
                 : mask ? reinterpret_cast<const void*>( trace3d_scout_kernel<true,0> ) : reinterpret_cast<const void*>( trace3d_scout_kernel<false,0> );
-        if ( zc_all( p ) > ZC_FEW && ( e = launch( k, ZC_SCOUTS, threads, full ) ) != hipSuccess ) return e;
+        if ( zc_all( p ) > ZC_FEW && zcell_decides( p.zc, p.n, p.Nz ) && ( e = launch( k, ZC_SCOUTS, threads, full ) ) != hipSuccess ) return e;
         p.zc.z_first = z_first;
     }
     else p.zc.route = nullptr;
@@ -865,7 +883,7 @@ hipError_t launch_trace3d_zcell( const trace3_params &p_in, uint32_t *tasks, hip
     const size_t lds = zcell_lds( p.zc.nzc, p.Nx * ( p.Ny + 3 ), p.zc.szp );
     if ( ( e = launch( k, uint32_t( grid ), threads, lds ) ) != hipSuccess ) return e;
     if ( tasks ) *tasks = uint32_t( grid ) * ( threads / WAVE );
-    if ( p.n == 0 || p.zc.nzc >= p.Nz ) return hipGetLastError();      // no window to leave
+    if ( p.n == 0 || ( p.zc.nzc >= p.Nz && p.zc.route == nullptr ) ) return hipGetLastError();      // no window to leave
     k = metrics ? zslice_kernel<MODE_METRICS>( mask, g16 ) : zslice_kernel<MODE_RHO>( mask, g16 );
     if ( ( e = launch( k, uint32_t( grid ), threads, full ) ) != hipSuccess ) return e;
     return hipGetLastError();
