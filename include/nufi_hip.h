@@ -218,7 +218,8 @@ int nufi_get_launch_shape(nufi_ctx *ctx, int *block, int *nodes_per_thread, int 
  * 64 threads, cuda_kernel.cu:123-124): times every built shape that fits the
  * LDS on the trace kernel at step n_probe over all nodes (`repeats` launches
  * each, HIP events on the context stream, history as currently on the device),
- * keeps the fastest and returns it.  Results are overwritten partials only. */
+ * keeps the fastest and returns it.  Results are overwritten partials only.
+ * 3D FP64 grids of the z-cell trace have one shape, which is timed and returned. */
 int nufi_autotune(nufi_ctx *ctx, uint64_t n_probe, int repeats, int *block, int *nodes_per_thread,
                   int *chunk, double *best_ms);
 

@@ -277,7 +277,7 @@ int effective_chunk( const nufi_ctx *c, const launch_shape &s, size_t *lds = nul
 
 // Default launch shapes (the autotuner refines them): 1D x-major 1024 threads
 // x 1 node (16 velocity rows per workgroup), the largest chunk two table
-// buffers in 160 KiB of LDS hold; 3D FP64 1024 threads x 2 nodes, FP32C 512 x 4.
+// buffers in 160 KiB of LDS hold; 3D FP64 512 threads x 8 nodes, FP32C 512 x 4.
 void default_shape( nufi_ctx *c )
 {
     const uint64_t waves = c->n_space * c->wpx;
@@ -308,7 +308,8 @@ void default_shape( nufi_ctx *c )
         int chunk = int( std::min<size_t>( c->lds_cap, 64 * 1024 ) / per );
         chunk = std::max( 1, std::min( chunk, 1 ) );
         // FP32C: the autotuner's pick on 16^3 x 32^3 (two 1-slice buffers); FP64:
-        // the z-cell kernel has one shape (512 x 8), its window kernel takes four for eight
+        // the z-cell kernel has one shape (512 x 8); the window kernel, which it is
+        // the pick of at 16^3, takes four for eight elsewhere
         if ( c->variant == TRACE_STRICT ) c->shape = launch_shape { 256, 1, chunk };
         else if ( c->variant == TRACE_FP32C ) c->shape = launch_shape { 512, 4, 1 };
         else c->shape = launch_shape { 512, 8, chunk };
@@ -1218,6 +1219,8 @@ int nufi_autotune( nufi_ctx *c, uint64_t n_probe, int repeats, int *block, int *
     else
     {
         if ( c->variant == TRACE_STRICT ) cand.push_back( { 256, 1, 1 } );
+        else if ( c->variant == TRACE_FAST && zcell_slices( c, n_probe ) )
+            cand.push_back( { 512, 8, 1 } );         // the z-cell trace has one shape: nothing to choose
         else
         {
             for ( int b : blocks1 ) for ( int np : npts ) for ( int ch : { 1, 2 } ) cand.push_back( { b, np, ch } );

@@ -159,3 +159,15 @@ def test_metrics_on_both_sides_of_the_wave_tasks(N, V):
             s.compute_metrics(17, a, b)
             s.download_metrics(parts)
         assert np.max(np.abs(parts - got) / np.abs(got)) <= 1e-13
+
+
+@pytest.mark.parametrize("N,V", GRIDS)
+def test_autotuner_has_nothing_to_choose_where_z_cells_trace(N, V):
+    """Every shape would time the same launches and the pick be noise."""
+    c = make(N, V)
+    with nufi.GpuScheduler(c) as s:
+        s.upload_history(history(c, 6, 0.0), 0, 6)
+        for shape in [(1024, 1, 1), (256, 2, 1)]:
+            s.set_launch_shape(*shape)
+            picked, ms = s.autotune(n_probe=6, repeats=1)
+            assert picked == (512, 8, 1) == s.launch_shape() and ms > 0
