@@ -101,7 +101,7 @@ inline uint32_t xm3_vgroup( uint64_t n_space, uint64_t n_vel )
 // The z-cell trace (trace3d_zcell.hip).  Velocity group g of w index iw: the
 // (u, v) indices g*vg .. g*vg+vg-1 (u innermost); its partial sum is
 // partials[(iw*ngw + g)*n_space + l].
-constexpr uint32_t ZCELL_PAIR2 = 48 * 1024, ZCELL_MAX = 4, ZCELL_MARKS = 1u << 16;
+constexpr uint32_t ZCELL_PAIR2 = 48 * 1024, ZCELL_MAX = 4;
 struct zcell_consts          // per axis: points, their inverse, drift in cells per unit velocity, kick constants
 {
     double N[3], iN[3], cd[3], kick[3], kickh[3];
@@ -259,7 +259,9 @@ hipError_t launch_trace3d( const trace3_params &p, int variant, const launch_sha
 zcell_plan plan_zcell( const nufi_config &g );
 // waves of a whole-grid metrics launch (its partials are four reals a wave)
 size_t zcell_metric_waves( const nufi_config &g, const zcell_plan &z );
-// workgroups (and their waves) of a whole-grid launch, at most ZCELL_MARKS; a mark each
+// workgroups (and their waves) of a whole-grid launch; a mark each.  A workgroup has
+// at least three partial sums to write on average (a plane has three points or more
+// and is cut into tiles of eight or more).
 size_t zcell_workgroups( const nufi_config &g, const zcell_plan &z, uint32_t *waves );
 hipError_t launch_trace3d_zcell( const trace3_params &p, uint32_t *tasks, hipStream_t st );
 // Whether a call of n slices lets the device choose between z-cells and whole

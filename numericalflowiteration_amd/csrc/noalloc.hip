@@ -1,8 +1,8 @@
 // noalloc.hip — nufi_rho3d_noalloc: rho of one 3D time step from a device
 // history the caller owns into a device rho the caller owns, with no device
 // allocation.  It runs the kernels of nufi_compute_rho on a 3D FP64 context
-// (the x-major fast trace of trace3d.hip, then the fixed-order partial sum of
-// field.hip), so its result equals compute_rho(n, 0, all nodes) followed by a
+// (the traces of trace3d_zcell.hip or trace3d.hip, chosen by the same rules, then
+// the fixed-order partial sum of field.hip), so its result equals compute_rho(n, 0, all nodes) followed by a
 // download into zeros, bit for bit.
 //
 // The rho partial sums (ppx partials per spatial point) go to `scratch`, one
@@ -25,7 +25,7 @@ namespace
 
 constexpr size_t SCRATCH_DOUBLES = NUFI_NOALLOC_SCRATCH_BYTES / sizeof(double);
 static __device__ __align__( 256 ) double scratch[SCRATCH_DOUBLES];
-static __device__ uint32_t marks[nufi_impl::ZCELL_MARKS];          // the z-cell trace's window marks
+static __device__ uint32_t marks[SCRATCH_DOUBLES / 3 + 1];         // the z-cell trace's window marks: one per three partial sums at most
 static __device__ nufi_impl::zcell_route route;                    // and route
 
 constexpr int MAX_DEVICES = 64;
@@ -93,6 +93,8 @@ extern "C" int nufi_rho3d_noalloc( const nufi_config *conf, uint64_t n, const do
         return fail( NUFI_ERR_UNSUPPORTED, "rho3d_noalloc: this grid needs " + std::to_string( std::max( ppw, ppx ) * n_space * 8 ) +
                                            " bytes of partial sums, above the " +
                                            std::to_string( NUFI_NOALLOC_SCRATCH_BYTES ) + "-byte scratch array" );
+    if ( zc.ok && zcell_workgroups( *conf, zc, nullptr ) > sizeof(marks) / sizeof(marks[0]) )
+        return fail( NUFI_ERR_UNSUPPORTED, "rho3d_noalloc: this grid needs more window marks than are held" );
     if ( st * sizeof(double) > 160 * 1024 )
         return fail( NUFI_ERR_UNSUPPORTED, "rho3d_noalloc: one slice of this grid exceeds the LDS" );
     const uint64_t wpx = ( n_vel + 63 ) / 64;

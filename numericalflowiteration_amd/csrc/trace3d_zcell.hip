@@ -827,7 +827,6 @@ zcell_plan plan_zcell( const nufi_config &g )
     }
     z.ok = z.vg > 0;
     z.ppx = uint32_t( z.ngw * g.Nw );
-    if ( z.ok && zcell_workgroups( g, z, nullptr ) > ZCELL_MARKS ) z.ok = false;      // nufi_rho3d_noalloc's marks
     return z;
 }
 

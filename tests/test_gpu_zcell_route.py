@@ -171,3 +171,25 @@ def test_autotuner_has_nothing_to_choose_where_z_cells_trace(N, V):
             s.set_launch_shape(*shape)
             picked, ms = s.autotune(n_probe=6, repeats=1)
             assert picked == (512, 8, 1) == s.launch_shape() and ms > 0
+
+
+def test_more_than_65536_workgroups():
+    """The z-cell trace takes grids of any number of workgroups, in a context and
+    without allocation (a mark per workgroup in either)."""
+    c = make((3, 3, 200), (6, 6, 400))
+    n = 4
+    hist = history(c, n, 0.1)
+    with nufi.GpuScheduler(c) as s:
+        s.upload_history(hist, 0, n)
+        rho = rho_of(s, n)
+        r = s.trace3d_route()
+        print(f"[route] {r}", flush=True)
+        assert r["zcell"] and r["workgroups"] > 65536
+        check_rho(c, n, hist, rho)
+    lib, rho_dev = _capi.load(), torch.zeros(c.n_space(), dtype=torch.float64, device="cuda")
+    h = torch.tensor(np.concatenate([hist, np.zeros(8)]), dtype=torch.float64, device="cuda")
+    rc = lib.nufi_rho3d_noalloc(ctypes.byref(c), n, ctypes.c_void_p(h.data_ptr()), h.numel(),
+                                ctypes.c_void_p(rho_dev.data_ptr()), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, lib.nufi_last_error(None)
+    torch.cuda.synchronize()
+    assert np.array_equal(rho_dev.cpu().numpy(), rho)
