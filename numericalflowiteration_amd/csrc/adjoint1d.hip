@@ -433,7 +433,7 @@ void adjoint_field_kernel( adjoint_field_params p )
     double2 *A = ldsa, *B = ldsa + 2*N, *tw = ldsa + 4*N;
     const uint32_t nt = twiddle_entries( N, p.log2x );
     for ( uint32_t i = threadIdx.x; i < nt; i += FIELD_BLOCK ) tw[i] = p.tw[i];
-    constexpr uint32_t PRE = 2;                              // the thread's first modes; N <= 2275 has up to 5
+    constexpr uint32_t PRE = 2;                              // the thread's first modes; N <= 2048 has up to 4
     double2 mu[PRE];
     double ew[PRE];
     #pragma unroll
@@ -494,7 +494,9 @@ void reduce_grad_kernel( const double *part, uint32_t n_tasks, uint32_t npar, do
 // Workgroups of 512 threads, 1024 where a CU would get two of them: one takes
 // the whole LDS.  Fewer workgroups add fewer global atomics (each adds to every
 // slice adjoint) and longer LDS queues: at 128 x 512, 256 threads (every CU)
-// 70 us, 512 (half of them) 65, 1024 103.  Two table buffers and padded adjoint rows where at least two slices of both fit.
+// 70 us, 512 (half of them) 65, 1024 103; above 131072 nodes, gradient to T = 5 by 512 /
+// 1024 threads: 133120 nodes 5.5 / 4.5 ms, 262144 7.7 / 5.7, 1048576 31.0 / 21.6 (velocity-
+// major 9.3, 11.4, 41.9).  Two table buffers and padded adjoint rows where at least two slices of both fit.
 void plan_adjoint1d( adjoint1_params &p, int n_cu, size_t lds_cap )
 {
     const uint64_t nodes = uint64_t( p.Nx ) * p.Nu;

@@ -7,7 +7,9 @@
 // half-kick with slice 0, and f0 at the foot.
 //
 // FP64 rho and metrics of grids whose z-cell window fits the LDS run in
-// trace3d_zcell.hip; launch_trace3d hands rho over.  Here:
+// trace3d_zcell.hip; launch_trace3d hands rho over, and takes it where that file's
+// deciding launches send a 16^3 history to the window kernel.  FP64 metrics of few
+// nodes, and of slices whose pads are no periodic copies, come here too.  Here:
 //
 // The workgroup streams coefficient slices through LDS (one slice is
 // (Nx+3)(Ny+3)(Nz+3) reals: 6859 = 54.9 KB FP64 at 16^3) and every node
