@@ -211,6 +211,12 @@ bool zcell_slices( const nufi_ctx *c, uint64_t n )
     return true;
 }
 
+// and whether rho of step n is
+bool zcell_step( const nufi_ctx *c, uint64_t n )
+{
+    return zcell_slices( c, n ) && zcell_rho( c->zc, n, c->conf, c->st );
+}
+
 // Whether the pads of a 3D slice (host) are the periodic copies.
 bool periodic_pads( const nufi_config &g, const double *s )
 {
@@ -237,13 +243,13 @@ void set_odd_pads( nufi_ctx *c, uint64_t n, bool odd )
 uint32_t rho_ppx( const nufi_ctx *c, uint64_t n )
 {
     const bool xm = c->variant == TRACE_FAST || ( c->dim == 1 && c->variant == TRACE_FP32C );
-    return xm ? ( zcell_slices( c, n ) ? c->zc.ppx : c->ppx ) : c->wpx;
+    return xm ? ( zcell_step( c, n ) ? c->zc.ppx : c->ppx ) : c->wpx;
 }
 
 // and those of the window kernel where step n may take it
 partial_alt rho_alt( const nufi_ctx *c, uint64_t n )
 {
-    if ( c->dim != 3 || c->variant != TRACE_FAST || !zcell_slices( c, n ) ) return partial_alt {};
+    if ( c->dim != 3 || c->variant != TRACE_FAST || !zcell_step( c, n ) ) return partial_alt {};
     return partial_alt { zcell_window( c->zc, n, c->conf.Nx, c->conf.Ny, c->conf.Nz ), c->ppx };
 }
 
@@ -375,7 +381,7 @@ int launch_trace( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_end, uin
         p.sy = c->sy; p.sz = c->sz; p.st = c->st; p.st32 = c->st32; p.wpx = c->wpx;
         p.l_first = uint32_t( l0 ); p.n_tasks = uint32_t( tasks );
         p.n_count = uint32_t( l1 - l0 + 1 ); p.vgroup = c->vgroup; p.ppx = c->ppx;
-        if ( zcell_slices( c, n ) ) p.zc = c->zc;
+        if ( zcell_step( c, n ) ) p.zc = c->zc;
         p.order = uint32_t( c->order );
         fill_trace3_geometry( p, c->conf );
         e = launch_trace3d( p, c->variant, c->shape, c->stream );
@@ -1219,7 +1225,7 @@ int nufi_autotune( nufi_ctx *c, uint64_t n_probe, int repeats, int *block, int *
     else
     {
         if ( c->variant == TRACE_STRICT ) cand.push_back( { 256, 1, 1 } );
-        else if ( c->variant == TRACE_FAST && zcell_slices( c, n_probe ) )
+        else if ( c->variant == TRACE_FAST && zcell_step( c, n_probe ) )
             cand.push_back( { 512, 8, 1 } );         // the z-cell trace has one shape: nothing to choose
         else
         {

@@ -313,6 +313,17 @@ inline bool fast3_dma( uint32_t chunk, uint32_t st )
 {
     return 2ull * ( uint64_t( chunk ) * st + 2 ) * sizeof(double) <= 160u * 1024u;
 }
+// Whether rho of step n is traced from z-cells and not by the window kernel.  With no
+// or one slice the passes' start and end are most of a call, and the window kernel's are
+// cheaper where it has the nodes to fill the chip (window / z-cells): n = 0 8^3 x 16^3 40 /
+// 68 us, 10^3 x 12^3 35 / 51, 20^3 x 24^3 1291 / 1678, but 4^3 x 8^3 31 / 19, 16^3 x 32^3
+// 1853 / 1663; n = 1, where two slices fit the LDS, 68 / 88, 62 / 74, 16^3 x 9^3 92 / 107,
+// 16^3 x 32^3 2573 / 2654, where not 20^3 3201 / 2829; from n = 2 on z-cells (10^3 92 / 91).
+inline bool zcell_rho( const zcell_plan &z, uint64_t n, const nufi_config &g, uint32_t st )
+{
+    if ( !z.ok || n > 1 || g.Nx * g.Ny * g.Nz * g.Nu * g.Nv * g.Nw < ( 1u << 19 ) ) return z.ok;
+    return n == 0 ? g.Nx == 16 && g.Ny == 16 && g.Nz == 16 : !fast3_dma( 1, st );
+}
 bool trace1d_shape_ok( int variant, int order, const launch_shape &s );
 // x-major fields (xw, rows, n_xt, ppx) and the threads of a workgroup from Nu,
 // ix_count and the shape; the grid of a launch (x-major or wave-task decomposition, by variant and mode) and the

@@ -87,7 +87,8 @@ extern "C" int nufi_rho3d_noalloc( const nufi_config *conf, uint64_t n, const do
     const uint64_t sy = conf->Nx + order - 1, sz = sy * ( conf->Ny + order - 1 ), st = sz * ( conf->Nz + order - 1 );
     const uint64_t n_space = conf->Nx * conf->Ny * conf->Nz, n_vel = conf->Nu * conf->Nv * conf->Nw;
     const uint32_t vgroup = xm3_vgroup( n_space, n_vel );
-    const zcell_plan zc = plan_zcell( *conf );
+    zcell_plan zc = plan_zcell( *conf );
+    zc.ok = zcell_rho( zc, n, *conf, uint32_t( st ) );
     const uint64_t ppw = ( n_vel + vgroup - 1 ) / vgroup, ppx = zc.ok ? zc.ppx : ppw;
     if ( std::max( ppw, ppx ) * n_space > SCRATCH_DOUBLES )
         return fail( NUFI_ERR_UNSUPPORTED, "rho3d_noalloc: this grid needs " + std::to_string( std::max( ppw, ppx ) * n_space * 8 ) +

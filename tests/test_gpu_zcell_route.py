@@ -193,3 +193,23 @@ def test_more_than_65536_workgroups():
     assert rc == 0, lib.nufi_last_error(None)
     torch.cuda.synchronize()
     assert np.array_equal(rho_dev.cpu().numpy(), rho)
+
+
+@pytest.mark.parametrize("N,V", [((8, 8, 8), (11, 9, 11)), ((8, 8, 8), (8, 8, 8)), ((16, 16, 16), (8, 8, 4)), ((20, 18, 20), (6, 6, 4))])
+def test_first_steps(N, V):
+    """rho of no, one and two slices, on both sides of the nodes at which the window
+    kernel takes the first two; without allocation the same bits."""
+    c = make(N, V)
+    hist = history(c, 3, 0.1)
+    lib, rho_dev = _capi.load(), torch.zeros(c.n_space(), dtype=torch.float64, device="cuda")
+    h = torch.tensor(np.concatenate([hist, np.zeros(8)]), dtype=torch.float64, device="cuda")
+    with nufi.GpuScheduler(c) as s:
+        s.upload_history(hist, 0, 3)
+        for n in (0, 1, 2):
+            rho = rho_of(s, n)
+            check_rho(c, n, hist, rho)
+            rc = lib.nufi_rho3d_noalloc(ctypes.byref(c), n, ctypes.c_void_p(h.data_ptr()), h.numel(),
+                                        ctypes.c_void_p(rho_dev.data_ptr()), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+            assert rc == 0, lib.nufi_last_error(None)
+            torch.cuda.synchronize()
+            assert np.array_equal(rho_dev.cpu().numpy(), rho)
