@@ -749,7 +749,9 @@ int nufi_compute_metrics( nufi_ctx *c, uint64_t n, uint64_t q_begin, uint64_t q_
             p.sy = c->sy; p.sz = c->sz; p.st = c->st; p.wpx = c->m_wpx;
             p.l_first = uint32_t( l0 ); p.n_tasks = uint32_t( tasks ); p.order = uint32_t( c->order );
             fill_trace3_geometry( p, g );
-            if ( variant == TRACE_FAST && zcell_metrics( c->zc, c->m_nodes, c->st ) && zcell_slices( c, n + 1 ) )
+            const uint64_t per_plane = g.Nx * g.Ny;
+            if ( variant == TRACE_FAST && zcell_slices( c, n + 1 ) &&
+                 zcell_metrics( g, c->zc, tasks, l1 / per_plane - l0 / per_plane + 1, c->st, c->n_cu ) )
             {
                 uint32_t waves = 0;
                 p.n_count = uint32_t( l1 - l0 + 1 ); p.zc = c->zc;

@@ -278,16 +278,26 @@ inline bool zcell_routed( const zcell_plan &z, uint64_t n, uint64_t Nz )
 {
     return z.ok && z.route != nullptr && ( z.check_pads ? n > 0 : zcell_decides( z, n, Nz ) );
 }
-// Whether the metrics of a grid are traced from z-cells (or whole slices in their
-// place) and not in wave tasks.  With less than a round of workgroups on the chip
-// a z-cell trace takes a round's time all the same (20 us a slice), wave tasks 15 to 21 ps
-// a node and slice while the slice they stage is small: n = 40, 4^3 x 8^3 289 / 80 us,
-// 6^3 x 8^3 410 / 105, 8^3 x 9^3 396 / 278, 8^3 x 12^3 777 / 571, 9x10x11 x 9x10x9 849 / 609;
-// above, 10^3 x 12^3 886 / 1184, 8^3 x 16^3 795 / 1090, 13x14x15 x 10^3 1392 / 2399.
-constexpr uint32_t WAVE_TASK_SLICE = 5120;      // reals
-inline bool zcell_metrics( const zcell_plan &z, uint64_t nodes, uint32_t st )
+// Whether a metrics call (`tasks` waves of wave tasks on `planes` z planes) is traced
+// from z-cells (or whole slices in their place) and not in wave tasks.  Either takes
+// so many rounds on the chip a slice.  z-cells: whole planes whatever part of them the
+// call asks for, a workgroup a CU, 9 us a round and pass of eight velocities, 11.4 where
+// axes wrap every step.  Wave tasks: as many workgroups of four waves as slices fit the
+// LDS, up to four, 3.5 us and 0.12 for each 1000 reals of the slice.  Wave tasks /
+// z-cells in us, n = 40: 4^3 x 8^3 80 / 289, 8^3 x 9^3 278 / 396, 8^3 x 12^3 571 / 777,
+// 10^3 x 12^3 1184 / 886, 8^3 x 16^3 1040 / 787 and an eighth of it 167 / 387, 16^3 x 9^3
+// 4148 / 1485, 1/8 of it 600 / 370, 1/16 318 / 370, 20 x 18 x 12 of 7 x 7 x 8 2730 / 945,
+// 1/8 391 / 471, 20^3 x 8^3 11600 / 2380, 1/16 640 / 480, 1/32 384 / 482; 16^3 x 32^3,
+// a quarter of a plane 2485 / 11150.
+constexpr uint32_t WAVE_TASK_SLICE = 5120;      // reals; see nufi_compute_metrics
+inline bool zcell_metrics( const nufi_config &g, const zcell_plan &z, uint64_t tasks, uint64_t planes, uint32_t st, int n_cu )
 {
-    return z.ok && !( nodes < ( 1u << 20 ) && st <= WAVE_TASK_SLICE );
+    if ( !z.ok ) return false;
+    const bool mask = ( g.Nx & ( g.Nx - 1 ) ) == 0 && ( g.Ny & ( g.Ny - 1 ) ) == 0 && ( g.Nz & ( g.Nz - 1 ) ) == 0;
+    const uint64_t cus = uint64_t( n_cu ), groups = zcell_workgroups( g, z, nullptr ) / g.Nz * planes;
+    const uint64_t held = std::min<uint64_t>( 4, 20480 / st ) * 4 * cus;
+    return ( mask ? 9.0 : 11.4 ) * double( ( z.vg + 7 ) / 8 ) * double( ( groups + cus - 1 ) / cus )
+         < ( 3.5 + 1.2e-4 * st ) * double( ( tasks + held - 1 ) / held );
 }
 // The flag by which the window kernel traces rho in the z-cell workgroups' place,
 // null where it never does.  At 16^3 its compiled strides and eight nodes a lane
@@ -318,7 +328,8 @@ inline bool fast3_dma( uint32_t chunk, uint32_t st )
 // cheaper where it has the nodes to fill the chip (window / z-cells): n = 0 8^3 x 16^3 40 /
 // 68 us, 10^3 x 12^3 35 / 51, 20^3 x 24^3 1291 / 1678, but 4^3 x 8^3 31 / 19, 16^3 x 32^3
 // 1853 / 1663; n = 1, where two slices fit the LDS, 68 / 88, 62 / 74, 16^3 x 9^3 92 / 107,
-// 16^3 x 32^3 2573 / 2654, where not 20^3 3201 / 2829; from n = 2 on z-cells (10^3 92 / 91).
+// 16^3 x 32^3 2573 / 2654, where not 20^3 3201 / 2829 (a 4-million-node one 130 / 147);
+// from n = 2 on z-cells (10^3 x 12^3 92 / 91, 10^3 x 16^3 183 / 214, 12^3 x 16^3 351 / 289).
 inline bool zcell_rho( const zcell_plan &z, uint64_t n, const nufi_config &g, uint32_t st )
 {
     if ( !z.ok || n > 1 || g.Nx * g.Ny * g.Nz * g.Nu * g.Nv * g.Nw < ( 1u << 19 ) ) return z.ok;

@@ -1,0 +1,36 @@
+"""Rules by the size of a call: 3D metrics of slabs (wave tasks) and of whole grids
+(z-cells) add up and hold against the oracle, at the 1e-12 of the other parity tests."""
+import numpy as np
+import pytest
+
+import numericalflowiteration_amd as nufi
+from numericalflowiteration_amd import config as C
+from tests import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+
+def wave3(c, n):
+    x, y, z = (np.arange(m + 3) % m * 2 * np.pi / m for m in (c.Nx, c.Ny, c.Nz))
+    return np.concatenate([0.04 * (np.cos(x + 0.1 * m)[None, None, :] + np.cos(y)[None, :, None] + np.cos(z - 0.2 * m)[:, None, None]).ravel()
+                           for m in range(n)])
+
+
+@pytest.mark.parametrize("N,V", [((16, 16, 16), (8, 6, 3)), ((20, 18, 12), (7, 7, 3)), ((8, 8, 8), (16, 8, 18)), ((13, 12, 9), (9, 8, 13))])
+def test_metrics_of_slabs_add_up(N, V):
+    c = C.config_3d(N, V, 1 / 8, 24.5 / 8, (0.0, 4 * np.pi), (-6.0, 6.0), C.F0_LANDAU_3D, alpha=0.05, k=0.5)
+    n, total = 17, c.n_nodes()
+    hist = wave3(c, n + 1)
+    with nufi.GpuScheduler(c) as s:
+        s.upload_history(hist, 0, n + 1)
+        whole = np.zeros(4)
+        s.compute_metrics(n)
+        s.download_metrics(whole)
+        for pieces in (2, 7, 29):
+            cuts, parts = np.linspace(0, total, pieces + 1).astype(np.int64), np.zeros(4)
+            for a, b in zip(cuts[:-1], cuts[1:]):
+                s.compute_metrics(n, int(a), int(b))
+                s.download_metrics(parts)
+            assert np.max(np.abs(parts - whole) / np.abs(whole)) <= 1e-13, pieces
+    ref = O.metrics(c, n, np.concatenate([hist, np.zeros(c.stride_t() + 8)]))
+    assert np.max(np.abs(whole - ref) / np.abs(ref)) <= 1e-12
