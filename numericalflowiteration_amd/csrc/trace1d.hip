@@ -658,7 +658,12 @@ static bool x_major( const trace1_params &p, int variant )
 // what counts is how many of them share a SIMD: the trace of 64 x 256 nodes at
 // n = 240 took 33.0 us in 16 workgroups of 16 waves and takes 24.2 in 64 of
 // 4; 128 x 512 at n = 160 30.6 -> 23.3; 100 x 515 at n = 160 (lanes of a
-// 64-wide tile no longer idle over 100 points either) 27.0 -> 19.9.
+// 64-wide tile no longer idle over 100 points either) 27.0 -> 19.9.  A quarter more
+// tiles at least, and tables of at most 16 KiB a slice: else the copies of more
+// workgroups and their waves of mixed rows cost more than the chip gives, and tiles
+// stay 64 wide, a narrower last one (n = 200, 64 wide / narrowed: 350 x 700 82.7 / 88.7
+// us, 700 x 330 64.1 / 73.6, 1500 x 48 108 / 119; n = 100, 3000 x 200, a quarter of its
+// x nodes 107 / 116; but 200 x 800 38.2 / 35.5, 130 x 900 35.3 / 31.6).
 // spread = false (a given block, batch launches): the tile count that leaves
 // the fewest lanes idle, the widest tile on ties.
 uint32_t trace1d_xm_setup( trace1_params &p, const launch_shape &s, bool spread, int n_cu )
@@ -670,7 +675,9 @@ uint32_t trace1d_xm_setup( trace1_params &p, const launch_shape &s, bool spread,
     if ( spread )
     {
         k = std::min( std::max( uint32_t( n_cu ) / p.ppx, k0 ), k1 );
-        p.xw = ( nx + k - 1 ) / k;
+        const size_t table = size_t( p.stride_q ) * ( p.qhist32 ? sizeof(float) : sizeof(double) );
+        if ( 4 * k < 5 * k0 || table > 16384 ) k = k0;
+        p.xw = k == k0 ? std::min( nx, 64u ) : ( nx + k - 1 ) / k;
         p.rows = XM_GROUP;
     }
     else

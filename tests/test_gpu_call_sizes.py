@@ -1,5 +1,6 @@
 """Rules by the size of a call: 3D metrics of slabs (wave tasks) and of whole grids
-(z-cells) add up and hold against the oracle, at the 1e-12 of the other parity tests."""
+(z-cells) add up and hold against the oracle, and 1D tiles with a narrower last one.
+The 1e-12 (FP64) and 1e-6 (FP32C) of the other parity tests."""
 import numpy as np
 import pytest
 
@@ -34,3 +35,27 @@ def test_metrics_of_slabs_add_up(N, V):
             assert np.max(np.abs(parts - whole) / np.abs(whole)) <= 1e-13, pieces
     ref = O.metrics(c, n, np.concatenate([hist, np.zeros(c.stride_t() + 8)]))
     assert np.max(np.abs(whole - ref) / np.abs(ref)) <= 1e-12
+
+
+# 64-wide tiles and 2, 1, 22 points more; tables past 16 KiB
+@pytest.mark.parametrize("prec,tol", [(nufi.FP64, 1e-12), (nufi.FP32C, 1e-6)])
+@pytest.mark.parametrize("Nx,Nu", [(130, 1400), (300, 1040), (65, 4100), (700, 60), (1500, 33)])
+def test_rho_tiles_and_partials(Nx, Nu, prec, tol):
+    c = C.config_1d(Nx, Nu, 1 / 16, 1.5, 0.0, 4 * np.pi, -10.0, 10.0, C.F0_LANDAU_1D, 0.05, 0.5)
+    n, st = 18, c.stride_t()
+    j = np.arange(st) % Nx
+    hist = np.concatenate([0.03 * np.cos(2 * np.pi * j / Nx + 0.2 * m) for m in range(n)])
+    cut = Nu * (Nx // 3) + 5
+    with nufi.GpuScheduler(c, precision=prec) as s:
+        s.upload_history(hist, 0, n)
+        whole, parts = np.zeros(Nx), np.zeros(Nx)
+        s.compute_rho(n)
+        s.download_rho(whole)
+        for a, b in ((0, cut), (cut, c.n_nodes())):
+            s.compute_rho(n, a, b)
+            s.download_rho(parts)
+    exact = O.rho(c, n, hist, exact_sum=True) - 1.0
+    for r in (whole, parts):
+        err = np.linalg.norm((r - r.mean()) - (exact - exact.mean())) / np.linalg.norm(exact - exact.mean())
+        print(f"[sizes] {Nx} x {Nu} {prec}: {err:.2e}", flush=True)
+        assert err <= tol
