@@ -42,11 +42,15 @@ namespace
 // Compensated sum over j < wpx of partials[j*n + i] by the G lanes of an
 // aligned group (field_sum_group), lane `part` taking j = part, part + G, ... in order; all
 // of them return it.  The loads go out up to RB at a time (clamped), so that a
-// sum waits for one round trip per RB G partials.
+// sum waits for one round trip per RB G partials.  ALONE: one lane a point (G = 1),
+// which takes 64 at a time in the reduction below (256 partials a point, 64 x 4096
+// nodes FP32C, n = 0: 19.9 -> 17.0 us; the field kernel has no room for it).
+template <uint32_t RB, bool ALONE>
 __device__ __forceinline__ double sum_partials( const double *__restrict__ partials, uint32_t wpx, size_t n,
-                                                uint32_t i, uint32_t part, uint32_t G )
+                                                uint32_t i, uint32_t part_, uint32_t G_ )
 {
-    constexpr uint32_t RB = 32, B = 8;
+    constexpr uint32_t B = 8;
+    const uint32_t G = ALONE ? 1u : G_, part = ALONE ? 0u : part_;
     csum acc { 0.0, 0.0 };
     for ( uint32_t j0 = 0; j0 < wpx; j0 += RB * G )
     {
@@ -197,7 +201,7 @@ __device__ __forceinline__ void field_body( const field_params &p, double2 *lds2
         const uint32_t G = p.sum_group, part = threadIdx.x & ( G - 1 ), wpx = partial_count( p.wpx, p.alt );
         for ( uint32_t i = threadIdx.x / G; i < N; i += FIELD_BLOCK / G )
         {
-            const double v = p.weight * sum_partials( p.partials, wpx, N, i, part, G );
+            const double v = p.weight * sum_partials<32,false>( p.partials, wpx, N, i, part, G );
             if ( part != 0 ) continue;
             if ( p.rho_out ) p.rho_out[i] = v;
             A[i] = make_double2( v, 0.0 );
@@ -291,14 +295,15 @@ void field_batch_kernel( const batch_field *__restrict__ runs, uint64_t n )
     else            field_body<false>( f, lds2b );
 }
 
+template <bool ALONE>
 __global__ __launch_bounds__( 64 ) void reduce_partials_kernel( const double *partials, uint32_t wpx, double weight,
                                         uint32_t first, uint32_t count, uint32_t n_space, uint32_t G, double *rho,
                                         partial_alt alt )
 {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, i = t / G, part = t & ( G - 1 );
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, i = ALONE ? t : t / G, part = ALONE ? 0u : t & ( G - 1 );
     if ( i >= n_space ) return;
     double v = 0.0;
-    if ( i >= first && i < first + count ) v = weight * sum_partials( partials, partial_count( wpx, alt ), n_space, i, part, G );
+    if ( i >= first && i < first + count ) v = weight * sum_partials<ALONE ? 64 : 32,ALONE>( partials, partial_count( wpx, alt ), n_space, i, part, G );
     if ( part == 0 ) rho[i] = v;
 }
 
@@ -432,7 +437,7 @@ hipError_t launch_reduce_partials( const double *partials, uint32_t wpx, double 
                                    double *rho, hipStream_t st, partial_alt alt )
 {
     const uint32_t block = 64, grid = ( n_space * G + block - 1 ) / block;     // a group per point, many CUs
-    hipLaunchKernelGGL( reduce_partials_kernel, dim3( grid ), dim3( block ), 0, st,
+    hipLaunchKernelGGL( ( G == 1 ? reduce_partials_kernel<true> : reduce_partials_kernel<false> ), dim3( grid ), dim3( block ), 0, st,
                         partials, wpx, weight, first, count, n_space, G, rho, alt );
     return hipGetLastError();
 }

@@ -1,6 +1,7 @@
 """Rules by the size of a call: 3D metrics of slabs (wave tasks) and of whole grids
-(z-cells) add up and hold against the oracle, and 1D tiles with a narrower last one.
-The 1e-12 (FP64) and 1e-6 (FP32C) of the other parity tests."""
+(z-cells) add up and hold against the oracle, 1D tiles with a narrower last one, and
+partial sums of one lane a point past 64 and its multiples.  The 1e-12 (FP64) and
+1e-6 (FP32C) of the other parity tests."""
 import numpy as np
 import pytest
 
@@ -37,9 +38,9 @@ def test_metrics_of_slabs_add_up(N, V):
     assert np.max(np.abs(whole - ref) / np.abs(ref)) <= 1e-12
 
 
-# 64-wide tiles and 2, 1, 22 points more; tables past 16 KiB
+# one lane a point with 64, 65, 130 partials; tables past 16 KiB; 64-wide tiles and 2, 1, 22 points more
 @pytest.mark.parametrize("prec,tol", [(nufi.FP64, 1e-12), (nufi.FP32C, 1e-6)])
-@pytest.mark.parametrize("Nx,Nu", [(130, 1400), (300, 1040), (65, 4100), (700, 60), (1500, 33)])
+@pytest.mark.parametrize("Nx,Nu", [(130, 1400), (257, 1024), (300, 1040), (65, 4100), (150, 2080), (700, 60), (1500, 33)])
 def test_rho_tiles_and_partials(Nx, Nu, prec, tol):
     c = C.config_1d(Nx, Nu, 1 / 16, 1.5, 0.0, 4 * np.pi, -10.0, 10.0, C.F0_LANDAU_1D, 0.05, 0.5)
     n, st = 18, c.stride_t()
