@@ -1,7 +1,8 @@
 """Rules by the size of a call: 3D metrics of slabs (wave tasks) and of whole grids
-(z-cells) add up and hold against the oracle, 1D tiles with a narrower last one, and
-partial sums of one lane a point past 64 and its multiples.  The 1e-12 (FP64) and
-1e-6 (FP32C) of the other parity tests."""
+(z-cells) add up and hold against the oracle, 1D tiles with a narrower last one, partial
+sums of one lane a point past 64 and its multiples, and transforms of lines without
+small factors, in four terms at a time and the rest.  The 1e-12 (FP64) and 1e-6 (FP32C)
+of the other parity tests."""
 import numpy as np
 import pytest
 
@@ -60,3 +61,16 @@ def test_rho_tiles_and_partials(Nx, Nu, prec, tol):
         err = np.linalg.norm((r - r.mean()) - (exact - exact.mean())) / np.linalg.norm(exact - exact.mean())
         print(f"[sizes] {Nx} x {Nu} {prec}: {err:.2e}", flush=True)
         assert err <= tol
+
+
+@pytest.mark.parametrize("prec", [nufi.FP64, nufi.FP32C])
+@pytest.mark.parametrize("Nx", [5, 6, 7, 11, 13, 22, 33, 97, 102, 721])
+def test_lines_without_small_factors(Nx, prec):
+    """Nodal values through the spline fit and back (FP32C contexts: the direct transform)."""
+    c = C.config_1d(Nx, 16, 1 / 16, 0.5, 0.0, 4 * np.pi, -10.0, 10.0, C.F0_LANDAU_1D, 0.05, 0.5)
+    v = np.cos(0.37 * np.arange(Nx)) + 0.2 * np.sin(1.1 * np.arange(Nx) + 0.5)
+    with nufi.GpuScheduler(c, precision=prec) as s:
+        a = np.asarray(s.interpolate(v)).ravel()[:Nx + 3]
+    back = (a[:Nx] + 4 * a[1:Nx + 1] + a[2:Nx + 2]) / 6
+    assert np.linalg.norm(back - v) <= 1e-12 * np.linalg.norm(v)
+    assert np.array_equal(a[Nx:], a[:3])
