@@ -323,17 +323,31 @@ inline bool fast3_dma( uint32_t chunk, uint32_t st )
 {
     return 2ull * ( uint64_t( chunk ) * st + 2 ) * sizeof(double) <= 160u * 1024u;
 }
-// Whether rho of step n is traced from z-cells and not by the window kernel.  With no
-// or one slice the passes' start and end are most of a call, and the window kernel's are
+// Whether rho of step n is traced from z-cells and not by the window kernel.  In the
+// first steps the passes' start and end are most of a call, and the window kernel's are
 // cheaper where it has the nodes to fill the chip (window / z-cells): n = 0 8^3 x 16^3 40 /
 // 68 us, 10^3 x 12^3 35 / 51, 20^3 x 24^3 1291 / 1678, but 4^3 x 8^3 31 / 19, 16^3 x 32^3
 // 1853 / 1663; n = 1, where two slices fit the LDS, 68 / 88, 62 / 74, 16^3 x 9^3 92 / 107,
-// 16^3 x 32^3 2573 / 2654, where not 20^3 3201 / 2829 (a 4-million-node one 130 / 147);
-// from n = 2 on z-cells (10^3 x 12^3 92 / 91, 10^3 x 16^3 183 / 214, 12^3 x 16^3 351 / 289).
+// 16^3 x 32^3 2573 / 2654.  Where they do not, and at n = 2 and 3, it is the rounds of
+// workgroups either takes, each on 256 CUs: the window kernel's of eight waves, a wave
+// four velocities a pass, 7 us and a slice 5 (7.8 where rows are short or wrap every
+// step, 9.6 with one buffer) a pass; z-cells' 7 us a round, 13 and a slice 8.4 or 9.8 a
+// pass.  n = 1 20^3 x 8^3 128 / 145, 20^3 x 14^3 705 / 609, 22^3 x 6^3 128 / 89; n = 2
+// 10^3 x 16^3 183 / 214, 32 x 8 x 8 of 64 x 8 x 2 73 / 84, 12^3 x 16^3 351 / 289; n = 3
+// 10^3 x 16^3 245 / 261, 16^3 x 16^3 653 / 605.
 inline bool zcell_rho( const zcell_plan &z, uint64_t n, const nufi_config &g, uint32_t st )
 {
-    if ( !z.ok || n > 1 || g.Nx * g.Ny * g.Nz * g.Nu * g.Nv * g.Nw < ( 1u << 19 ) ) return z.ok;
-    return n == 0 ? g.Nx == 16 && g.Ny == 16 && g.Nz == 16 : !fast3_dma( 1, st );
+    const uint64_t space = g.Nx * g.Ny * g.Nz, vel = g.Nu * g.Nv * g.Nw;
+    if ( !z.ok || n > 3 || space * vel < ( 1u << 19 ) ) return z.ok;
+    if ( n == 0 ) return g.Nx == 16 && g.Ny == 16 && g.Nz == 16;
+    const bool two = fast3_dma( 1, st );
+    if ( n == 1 && two ) return false;
+    const bool mask = ( g.Nx & ( g.Nx - 1 ) ) == 0 && ( g.Ny & ( g.Ny - 1 ) ) == 0 && ( g.Nz & ( g.Nz - 1 ) ) == 0;
+    const uint64_t vg = xm3_vgroup( space, vel ), groups = ( space + 63 ) / 64 * ( ( ( vel + vg - 1 ) / vg + 7 ) / 8 );
+    const double w = double( ( groups + 255 ) / 256 * ( vg / 4 ) ) * ( double( n ) * ( !two ? 9.6 : mask && g.Nx >= 16 ? 5.0 : 7.8 ) + 7.0 );
+    const double c = double( ( zcell_workgroups( g, z, nullptr ) + 255 ) / 256 )
+                   * ( double( ( z.vg + 7 ) / 8 ) * ( double( n ) * ( mask ? 8.4 : 9.8 ) + 13.0 ) + 7.0 );
+    return c <= w;
 }
 bool trace1d_shape_ok( int variant, int order, const launch_shape &s );
 // x-major fields (xw, rows, n_xt, ppx) and the threads of a workgroup from Nu,

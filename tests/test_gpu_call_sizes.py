@@ -1,12 +1,16 @@
 """Rules by the size of a call: 3D metrics of slabs (wave tasks) and of whole grids
 (z-cells) add up and hold against the oracle, 1D tiles with a narrower last one, partial
 sums of one lane a point past 64 and its multiples, and transforms of lines without
-small factors, in four terms at a time and the rest.  The 1e-12 (FP64) and 1e-6 (FP32C)
+small factors, in four terms at a time and the rest; 3D rho of the first steps.  The 1e-12 (FP64) and 1e-6 (FP32C)
 of the other parity tests."""
+import ctypes
+
 import numpy as np
 import pytest
+import torch                  # before the library: one HIP runtime for both
 
 import numericalflowiteration_amd as nufi
+from numericalflowiteration_amd import _capi
 from numericalflowiteration_amd import config as C
 from tests import oracle_lib as O
 
@@ -74,3 +78,28 @@ def test_lines_without_small_factors(Nx, prec):
     back = (a[:Nx] + 4 * a[1:Nx + 1] + a[2:Nx + 2]) / 6
     assert np.linalg.norm(back - v) <= 1e-12 * np.linalg.norm(v)
     assert np.array_equal(a[Nx:], a[:3])
+
+
+@pytest.mark.parametrize("N,V", [((32, 8, 8), (64, 8, 2)), ((16, 8, 8), (20, 16, 5)), ((10, 9, 10), (16, 16, 9)), ((20, 20, 20), (8, 8, 2)),
+                                 ((12, 12, 12), (8, 8, 6))])
+def test_first_steps_3d(N, V):
+    """rho of up to four slices by whichever kernel; without allocation the same bits."""
+    c = C.config_3d(N, V, 1 / 8, 24.5 / 8, (0.0, 4 * np.pi), (-6.0, 6.0), C.F0_LANDAU_3D, alpha=0.05, k=0.5)
+    hist = wave3(c, 4)
+    pts = np.unique(np.linspace(0, c.n_space() - 1, 12).astype(np.int64))
+    lib, rho_dev = _capi.load(), torch.zeros(c.n_space(), dtype=torch.float64, device="cuda")
+    h = torch.tensor(np.concatenate([hist, np.zeros(8)]), dtype=torch.float64, device="cuda")
+    with nufi.GpuScheduler(c) as s:
+        s.upload_history(hist, 0, 4)
+        for n in (1, 2, 3, 4):
+            rho = np.zeros(c.n_space())
+            s.compute_rho(n)
+            s.download_rho(rho)
+            ref = O.rho3d_points(c, n, hist, pts, exact_sum=True)
+            ref = ref - ref.mean() + rho[pts].mean()          # the oracle's constant ("+1") aside
+            assert np.linalg.norm(rho[pts] - ref) <= 1e-12 * np.linalg.norm(ref)
+            rc = lib.nufi_rho3d_noalloc(ctypes.byref(c), n, ctypes.c_void_p(h.data_ptr()), h.numel(),
+                                        ctypes.c_void_p(rho_dev.data_ptr()), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+            assert rc == 0, lib.nufi_last_error(None)
+            torch.cuda.synchronize()
+            assert np.array_equal(rho_dev.cpu().numpy(), rho)
