@@ -84,7 +84,7 @@ __device__ __forceinline__ double sum_partials( const double *__restrict__ parti
 constexpr uint32_t FIELD_EBUF_MAX = 1024;
 __host__ __device__ inline uint32_t field_ebuf( uint32_t N ) { return N <= FIELD_EBUF_MAX ? ( N + 1 ) & ~1u : 0u; }
 
-__device__ double2 *fft3( double2 *A, double2 *B, const field_params &p, const double2 *tx, const double2 *ty,
+__device__ __forceinline__ double2 *fft3( double2 *A, double2 *B, const field_params &p, const double2 *tx, const double2 *ty,
                           const double2 *tz, bool inverse )
 {
     if ( p.N == p.Nx )
