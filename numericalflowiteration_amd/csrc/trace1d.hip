@@ -141,7 +141,7 @@ __device__ __forceinline__ xm_node make_xm_node( const trace1_params &p, const x
 // f of the workgroup's nodes -> LDS -> one compensated sum per (x, group of
 // XM_GROUP consecutive velocities), summed in iu order, at partials[group*Nx + x].  `fbuf` may alias the
 // history chunk: the barrier below ends its use.
-template <int NPT>
+template <int NPT, int BLOCK>
 __device__ __forceinline__ void xm_reduce( const trace1_params &p, const xm_tile &t, const xm_node id[NPT],
                                            const double f[NPT], double *fbuf )
 {
@@ -153,7 +153,7 @@ __device__ __forceinline__ void xm_reduce( const trace1_params &p, const xm_tile
         for ( int r = 0; r < NPT; ++r ) fbuf[ id[r].vi * p.xw + t.xo ] = id[r].active ? f[r] : 0.0;
     }
     __syncthreads();
-    for ( uint32_t k = threadIdx.x; k < groups * p.xw; k += blockDim.x )
+    for ( uint32_t k = threadIdx.x; k < groups * p.xw; k += BLOCK > 0 ? uint32_t( BLOCK ) : blockDim.x )
     {
         const uint32_t xo = k % p.xw, gi = k / p.xw;
         const uint32_t xl = t.xt * p.xw + xo, gg = t.vb * groups + gi;
@@ -362,7 +362,7 @@ __device__ __forceinline__ void trace1d_poly_body( const trace1_params &p, uint3
     double f[NPT];
     #pragma unroll
     for ( int r = 0; r < NPT; ++r ) f[r] = id[r].active ? f0_1d( p.f0, p.x_min + s[r]*p.dx, u[r] ) : 0.0;
-    xm_reduce<NPT>( p, tile, id, f, lds );
+    xm_reduce<NPT,BLOCK>( p, tile, id, f, lds );
 }
 
 // BLOCK = 0: any workgroup size up to the limit (512 with four nodes a
@@ -488,7 +488,7 @@ __device__ __forceinline__ void trace1d_fp32c_body( const trace1_params &p, uint
         const double u = fp32c_velocity( fr, uh[r], ul[r] ) / cd;
         f[r] = id[r].active ? f0_1d( p.f0, p.x_min + s*p.dx, u ) : 0.0;
     }
-    xm_reduce<NPT>( p, tile, id, f, reinterpret_cast<double*>( ldsf ) );
+    xm_reduce<NPT,BLOCK>( p, tile, id, f, reinterpret_cast<double*>( ldsf ) );
 }
 
 template <int NPT, bool POW2, int BLOCK>
@@ -658,12 +658,13 @@ static bool x_major( const trace1_params &p, int variant )
 // what counts is how many of them share a SIMD: the trace of 64 x 256 nodes at
 // n = 240 took 33.0 us in 16 workgroups of 16 waves and takes 24.2 in 64 of
 // 4; 128 x 512 at n = 160 30.6 -> 23.3; 100 x 515 at n = 160 (lanes of a
-// 64-wide tile no longer idle over 100 points either) 27.0 -> 19.9.  A quarter more
-// tiles at least, and tables of at most 16 KiB a slice: else the copies of more
-// workgroups and their waves of mixed rows cost more than the chip gives, and tiles
-// stay 64 wide, a narrower last one (n = 200, 64 wide / narrowed: 350 x 700 82.7 / 88.7
-// us, 700 x 330 64.1 / 73.6, 1500 x 48 108 / 119; n = 100, 3000 x 200, a quarter of its
-// x nodes 107 / 116; but 200 x 800 38.2 / 35.5, 130 x 900 35.3 / 31.6).
+// 64-wide tile no longer idle over 100 points either) 27.0 -> 19.9.  Tiles of
+// 48 x nodes at most (12 waves, three a SIMD; wider ones leave some SIMD its four), and
+// tables of at most 16 KiB a slice: else the copies of more workgroups and their waves
+// of mixed rows cost more than they give, and tiles stay 64 wide, a narrower last one
+// (n = 200, 64 wide / narrowed: 350 x 700 82.7 / 88.7 us, 700 x 330 64.1 / 73.6, 256 x 800
+// at n = 800 FP32C 112.5 / 117.5, 1500 x 48 108 / 119; n = 100, 3000 x 200, a quarter of
+// its x nodes 107 / 116; but 200 x 800 38.2 / 35.5, 130 x 900 35.3 / 31.6).
 // spread = false (a given block, batch launches): the tile count that leaves
 // the fewest lanes idle, the widest tile on ties.
 uint32_t trace1d_xm_setup( trace1_params &p, const launch_shape &s, bool spread, int n_cu )
@@ -676,8 +677,8 @@ uint32_t trace1d_xm_setup( trace1_params &p, const launch_shape &s, bool spread,
     {
         k = std::min( std::max( uint32_t( n_cu ) / p.ppx, k0 ), k1 );
         const size_t table = size_t( p.stride_q ) * ( p.qhist32 ? sizeof(float) : sizeof(double) );
-        if ( 4 * k < 5 * k0 || table > 16384 ) k = k0;
-        p.xw = k == k0 ? std::min( nx, 64u ) : ( nx + k - 1 ) / k;
+        p.xw = ( nx + k - 1 ) / k;
+        if ( p.xw > 48 || table > 16384 ) p.xw = std::min( nx, 64u );
         p.rows = XM_GROUP;
     }
     else
