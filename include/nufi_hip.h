@@ -231,7 +231,8 @@ int nufi_autotune(nufi_ctx *ctx, uint64_t n_probe, int repeats, int *block, int 
  * cells; out[3]: what nodes outside their window were found to cost, in 1/65536
  * of a workgroup's trace (0 where the bound settled it); out[4]: workgroups
  * redone from whole slices; out[5]: workgroups.  Calls of fewer than 16 slices
- * decide nothing and leave out[1..3] as they were.
+ * decide nothing and leave out[1..3] as they were; calls that other kernels
+ * trace (the first steps of many nodes, metrics of few) leave all of it.
  */
 int nufi_trace3d_route(nufi_ctx *ctx, uint64_t out[6]);
 
